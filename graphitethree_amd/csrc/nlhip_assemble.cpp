@@ -100,22 +100,11 @@ System* lscm_create(uint32_t nv, const double* points, uint32_t nt, const uint32
     LSRows rows;
     lscm_rows_device(nv, P, nt, T, rows, s);
     const uint32_t nvars = 2 * nv;
-    std::vector<uint32_t> h_free(nvars);
-    std::vector<double> h_values(nvars, 0.0);
-    uint32_t nfree = 0;
-    for (uint32_t v = 0; v < nvars; ++v) {
-        const bool lk = (v / 2 == pin[0]) || (v / 2 == pin[1]);
-        h_free[v] = lk ? 0xffffffffu : nfree++;
-    }
-    h_values[2 * pin[0]] = uv[0];
-    h_values[2 * pin[0] + 1] = uv[1];
-    h_values[2 * pin[1]] = uv[2];
-    h_values[2 * pin[1] + 1] = uv[3];
+    const uint32_t nfree = nvars - 4;
     if (nfree_out) *nfree_out = nfree;
     DevBuf<uint32_t> d_free(nvars);
     DevBuf<double> d_values(nvars);
-    copy_in(d_free.get(), h_free.data(), size_t(nvars) * 4, s);
-    copy_in(d_values.get(), h_values.data(), size_t(nvars) * 8, s);
+    lscm_free_device(nv, pin, uv, d_free.get(), d_values.get(), s);
     LSInput in;
     in.nrows = rows.nrows;
     in.nvars = nvars;

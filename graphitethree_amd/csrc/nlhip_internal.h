@@ -562,6 +562,10 @@ struct LSRows {
 };
 void lscm_rows_device(uint32_t nv, const double* points, uint32_t nt, const uint32_t* triangles,
                       LSRows& rows, hipStream_t s);
+// Free indices (0xffffffff: locked) and locked values of the 2 nv variables of
+// an LSCM mesh with the two vertices pin[] at (uv[0], uv[1]), (uv[2], uv[3]).
+void lscm_free_device(uint32_t nv, const uint32_t pin[2], const double uv[4],
+                      uint32_t* free_index, double* values, hipStream_t s);
 // Throws when a triangle's vertices lie in different charts (device arrays;
 // chart c owns vertices [voff[c], voff[c+1])).
 void check_triangle_charts(uint32_t nt, const uint32_t* T, const uint32_t* voff, uint32_t nc,

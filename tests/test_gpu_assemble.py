@@ -288,3 +288,39 @@ def test_atlas_rejects_bad_charts(hip):
     vo2[1] = 2                                 # a chart of two vertices
     with pytest.raises(capi.NLHIPError):
         capi.Batch.lscm_atlas(vo2, P, T, pins, uv)
+
+
+@pytest.mark.parametrize("occ,length,cols", [(1, 1, 1), (64, 2, 64), (64, 2, 65), (65, 2, 20),
+                                             (3, 64, 64), (2, 65, 65), (22, 3, 64), (40, 5, 33),
+                                             (63, 1, 1)])
+def test_limits_of_the_plan_by_variable(hip, occ, length, cols):
+    """Variable 5 in `occ` entries of rows of `length` entries with `cols`
+    distinct columns: one wavefront holds up to 64 of each, more takes the
+    sorted plan; both give the context's bits (repeats, zeros of either sign,
+    locked variables and empty rows among them)."""
+    rng = np.random.default_rng(occ * 1000 + length * 10 + cols)
+    nvars = 200
+    others = 5 + 1 + rng.permutation(nvars - 6)[:max(cols - 1, 0)]
+    rows, left = [], list(others)
+    for _ in range(occ):
+        row = [5]
+        while len(row) < length:
+            row.append(left.pop() if left else int(rng.choice(others)) if len(others) else 5)
+        rng.shuffle(row)
+        rows.append(row)
+    for i in range(60):  # a few more, and empty ones
+        rows.insert(int(rng.integers(0, len(rows) + 1)),
+                    list(rng.choice([v for v in range(nvars) if v != 5], i % 4)))
+    rp = np.cumsum([0] + [len(r) for r in rows]).astype(np.uint32)
+    var = np.concatenate([np.asarray(r, dtype=np.int64) for r in rows]).astype(np.uint32)
+    coef = rng.standard_normal(len(var))
+    coef[rng.random(len(var)) < 0.1] = -0.0
+    locked = np.zeros(nvars, dtype=np.uint8)
+    locked[[0, 199]] = 1
+    values = rng.standard_normal(nvars)
+    rhs = rng.standard_normal(len(rows))
+    S, b = capi.System.least_squares(nvars, rp, var, coef, row_rhs=rhs, locked=locked,
+                                     values=values)
+    crs, b_ref = oracle_system(nvars, rp, var, coef, rhs, locked, values)
+    assert_same(S, b[0], crs, b_ref)
+    S.close()
