@@ -17,10 +17,62 @@ constexpr uint32_t kNumXcd = 8;       // MI355X: 8 XCDs, each with its own L2
 
 // Sum over each aligned group of W lanes (W a power of two <= 64).  A xor
 // butterfly: every lane of the group ends with the same, fixed-order sum.
+// The lanes of a group exchange by DPP within rows of 16 and by gfx950's row
+// swaps across them (a sum is the same from either side of an exchange):
+// an exchange through LDS permutes (__shfl_xor) costs some 130 cycles, these a
+// few, and six follow one another in every wavefront's sum.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_word(uint32_t v) {
+    return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), CTRL, 0xf, 0xf, true));
+}
+template <int O>
+__device__ __forceinline__ uint32_t xor_word(uint32_t v) {
+    static_assert(O == 1 || O == 2 || O == 4 || O == 8, "within a row of 16 lanes");
+    if constexpr (O == 1) return dpp_word<0xB1>(v);         // quad_perm 1,0,3,2
+    else if constexpr (O == 2) return dpp_word<0x4E>(v);    // quad_perm 2,3,0,1
+    else if constexpr (O == 4) return dpp_word<0x1B>(dpp_word<0x141>(v));  // xor 7, xor 3
+    else return dpp_word<0x128>(v);                         // row_ror 8
+}
+template <int O>
+__device__ __forceinline__ float xor_add(float v) {
+    const uint32_t b = __float_as_uint(v);
+    if constexpr (O == 32) {
+        const auto s = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+        return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+    } else if constexpr (O == 16) {
+        const auto s = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+        return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+    } else {
+        return v + __uint_as_float(xor_word<O>(b));
+    }
+}
+template <int O>
+__device__ __forceinline__ double xor_add(double v) {
+    const uint64_t b = uint64_t(__double_as_longlong(v));
+    const uint32_t lo = uint32_t(b), hi = uint32_t(b >> 32);
+    auto join = [](uint32_t l, uint32_t h) {
+        return __longlong_as_double((long long)((uint64_t(h) << 32) | l));
+    };
+    if constexpr (O == 32) {
+        const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        return join(l[0], h[0]) + join(l[1], h[1]);
+    } else if constexpr (O == 16) {
+        const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        return join(l[0], h[0]) + join(l[1], h[1]);
+    } else {
+        return v + join(xor_word<O>(lo), xor_word<O>(hi));
+    }
+}
 template <int W, typename T>
 __device__ __forceinline__ T group_sum(T v) {
-#pragma unroll
-    for (int o = W / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, W);
+    if constexpr (W > 32) v = xor_add<32>(v);
+    if constexpr (W > 16) v = xor_add<16>(v);
+    if constexpr (W > 8) v = xor_add<8>(v);
+    if constexpr (W > 4) v = xor_add<4>(v);
+    if constexpr (W > 2) v = xor_add<2>(v);
+    if constexpr (W > 1) v = xor_add<1>(v);
     return v;
 }
 

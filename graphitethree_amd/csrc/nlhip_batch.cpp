@@ -159,7 +159,9 @@ void batch_loop(Batch& B, BatchWork<T>& w, bool precond, int max_iter, uint32_t 
         return k;
     };
     uint32_t pgrid = 0;
+    std::unique_lock<std::mutex> barrier_lock(grid_barrier_mutex(), std::defer_lock);
     if (B.persistent) {
+        barrier_lock.lock();
         NLHIP_CHECK(batch_persistent_grid<T>(w.args, precond, &pgrid));
         pgrid = std::min(pgrid, std::max(B.grid, 1u));
     } else {

@@ -123,6 +123,11 @@ std::shared_mutex& capture_mutex() {
     return *m;
 }
 
+std::mutex& grid_barrier_mutex() {
+    static std::mutex* m = new std::mutex();  // process lifetime
+    return *m;
+}
+
 Stream::Stream() {
     device();
     auto g = no_capture_guard();

@@ -215,6 +215,10 @@ class Event {
 
 float elapsed_ms(const Event& a, const Event& b);
 
+// Held while a kernel with grid-wide barriers may be running: two of them,
+// each partly resident, would wait for one another.
+std::mutex& grid_barrier_mutex();
+
 // ------------------------------------------------------------------ graphs
 
 // A captured sequence of launches replayed as one hipGraph.
@@ -352,6 +356,10 @@ struct CGWorkspace {
     DevBuf<T> x, b, r, h, d, q, part;
     DevBuf<CGStatus<T>> st;
     PinnedBuf<CGStatus<T>> st_host;  // two slots
+    DevBuf<T> dh;                    // scratch of the iterations in one launch
+    DevBuf<uint64_t> slots;
+    DevBuf<uint32_t> bar;
+    PinnedBuf<uint32_t> bar_host;
     GraphLadder graph;
     int graph_rpw = 0;
     bool graph_precond = false;

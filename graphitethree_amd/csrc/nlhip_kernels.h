@@ -180,6 +180,31 @@ hipError_t cg_step(const CGArgs<T>& a, int rpw, bool precond, hipStream_t s);
 template <typename T>
 hipError_t cg_step_part(const CGArgs<T>& a, int rpw, bool precond, int part, hipStream_t s);
 
+// Many iterations per launch (k_cg_persist.hip) for systems whose matrix fits
+// in registers.
+constexpr uint32_t kPersistBarPad = 32;          // words between barrier counters
+constexpr uint32_t kPersistFail = 0x80000000u;   // bit of bar[0]: a wait was given up
+constexpr int kPersistSmall = 1, kPersistRows = 2, kPersistBlocks = 3;
+template <typename T>
+struct CGPersist {
+    int kind;          // 0: not for this system
+    uint32_t wgs;      // workgroups that take part
+    uint32_t stride;   // every stride-th workgroup of the grid does
+    uint32_t threads;  // per workgroup
+    uint32_t n_iter;   // iterations of this launch
+    T* dh;             // 2 m: (d, h) of every row
+    uint64_t* slots;   // persist_slot_words(P): tagged d.q, r.h and r.r partials
+    uint32_t* bar;     // 9 kPersistBarPad words: root counter, one per XCD
+};
+template <typename T>
+constexpr uint32_t persist_slot_words(uint32_t P) {
+    return 3u * P * uint32_t(sizeof(T) / 4);
+}
+template <typename T>
+void cg_persist_plan(const CGArgs<T>& a, int code, uint32_t cus, CGPersist<T>& p);
+template <typename T>
+hipError_t cg_persist(const CGArgs<T>& a, const CGPersist<T>& p, hipStream_t s);
+
 // ---- batched systems (k_batch.hip) ----------------------------------------
 
 // A batch tile is 4 passes of 64 rows, or of 64 block rows (row pairs) for

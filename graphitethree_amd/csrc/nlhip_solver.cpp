@@ -225,6 +225,8 @@ void CGWorkspace<T>::ensure(uint32_t n_, uint32_t P_) {
     part.alloc(size_t(kSpmvGridMul + 3) * P);  // d.q (up to kSpmvGridMul P), r.h, r.r, b.b
     st.alloc(1);
     st_host.ensure(2);
+    dh.release();
+    slots.release();
 }
 template struct CGWorkspace<double>;
 template struct CGWorkspace<float>;
@@ -279,12 +281,52 @@ uint32_t auto_check_every(const System& S) {
     return uint32_t(std::clamp(2.0e-3 / iter_s, 8.0, 128.0));
 }
 
-// Runs the captured iterations of a started CG (arguments set, status open)
-// until the device-side loop has stopped; `budget` bounds the iterations it
-// can still run.  Returns the final status.
+// Iterations of one k_cg_persist launch (some 10 ms).
+constexpr uint32_t kPersistIters = 4096;
+
+// Runs a started CG (arguments set, status open) with many iterations per
+// launch until its loop has stopped (the status in fin).  False where the
+// system is not of that kind, another such kernel holds the device, or a
+// grid-wide wait was given up: the state is then where the captured
+// iterations, which form the same sums, continue.
+template <typename T>
+static bool run_persist(System& S, CGWorkspace<T>& ws, CGStatus<T>& fin) {
+    if (direct_launches()) return false;
+    CGPersist<T> p{};
+    cg_persist_plan<T>(ws.args, ws.code, uint32_t(std::max(0, device().cu_count)), p);
+    if (!p.kind) return false;
+    std::unique_lock<std::mutex> lock(grid_barrier_mutex(), std::try_to_lock);
+    if (!lock.owns_lock()) return false;
+    hipStream_t s = S.stream.get();
+    ws.dh.ensure(2 * size_t(S.n));
+    ws.slots.ensure(persist_slot_words<T>(ws.args.P));
+    ws.bar.ensure(9 * kPersistBarPad);
+    ws.bar_host.ensure(1);
+    p.n_iter = kPersistIters;
+    p.dh = ws.dh.get();
+    p.slots = ws.slots.get();
+    p.bar = ws.bar.get();
+    CGStatus<T>* host = ws.st_host.get();
+    for (;;) {
+        NLHIP_CHECK(cg_persist<T>(ws.args, p, s));
+        NLHIP_CHECK(hipMemcpyAsync(host, ws.st.get(), sizeof(CGStatus<T>), hipMemcpyDeviceToHost, s));
+        NLHIP_CHECK(hipMemcpyAsync(ws.bar_host.get(), p.bar, 4, hipMemcpyDeviceToHost, s));
+        S.stream.sync();
+        if (ws.bar_host.get()[0] & kPersistFail) return false;
+        if (host[0].done) break;
+    }
+    fin = host[0];
+    return true;
+}
+
+// Runs the iterations of a started CG (arguments set, status open), captured
+// or many to a launch, until the device-side loop has stopped; `budget`
+// bounds the iterations it can still run.  Returns the final status.
 template <typename T>
 static CGStatus<T> run_ladder(System& S, CGWorkspace<T>& ws, bool precond, uint32_t K,
                               uint64_t budget) {
+    CGStatus<T> last;
+    if (run_persist<T>(S, ws, last)) return last;
     hipStream_t s = S.stream.get();
     if (ws.graph_rpw != ws.code || ws.graph_precond != precond ||
         std::memcmp(&ws.graph_args, &ws.args, sizeof(CGArgs<T>)) != 0)

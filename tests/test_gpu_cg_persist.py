@@ -1,0 +1,102 @@
+"""The PCG with many iterations per launch (systems whose matrix fits in the
+registers of the resident workgroups): the bits, iteration counts and
+residuals of the three launches per iteration, which the same solves run in a
+process that enqueues every launch directly (NLHIP_DIRECT_LAUNCH=1)."""
+import hashlib
+import json
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+from graphitethree_amd import capi
+from graphitethree_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+def random_spd(n, deg, seed, pairs=False):
+    """Symmetric, diagonally dominant, 0 to `deg` random neighbours per row
+    (some rows only their diagonal); pairs: each entry a 2x2 block."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(seed)
+    m = n // 2 if pairs else n
+    k = rng.integers(0, deg // 2 + 1, m)
+    r = np.repeat(np.arange(m), k)
+    c = np.clip(r + rng.integers(-300, 301, len(r)), 0, m - 1)
+    A = sp.coo_matrix((rng.standard_normal(len(r)), (r, c)), shape=(m, m)).tocsr()
+    A = A + A.T
+    A = A + sp.diags(np.asarray(abs(A).sum(axis=1)).ravel() + 0.1)
+    if pairs:
+        A = sp.kron(A, np.array([[2.0, 0.5], [0.5, 1.0]]))
+    A = A.tocsr()
+    A.sort_indices()
+    return W.SystemCRS(A.indptr.astype(np.uint32), A.indices.astype(np.uint32), A.data,
+                       rng.standard_normal((1, n)))
+
+
+def cases():
+    chart = lambda nv: W.lscm_system(W.chart_mesh(nv, 3))  # noqa: E731
+    lap = lambda k: W.cotan_system(W.grid_mesh(k, 2), t=1.0, nrhs=1)  # noqa: E731
+    c = [("one_row", random_spd(1, 0, 1), {}, {}), ("two_rows", random_spd(2, 2, 1), {}, {}),
+         ("lap_8", lap(8), {}, {}), ("lap_no_precond", lap(70), {}, dict(precond="none")),
+         ("u32_columns", lap(64), dict(offsets=False), {}),
+         ("cap", chart(3000), {}, dict(max_iter=7)),
+         ("cap_0", chart(300), {}, dict(max_iter=0)),
+         ("no_confirm", chart(1000), {}, dict(confirm=0)),
+         ("tight", chart(2000), {}, dict(eps=3e-13, max_iter=3000)),
+         ("mixed_small", lap(90), dict(fp32=True), dict(precision="mixed")),
+         ("mixed_rows", lap(200), dict(fp32=True), dict(precision="mixed")),
+         ("mixed_blocks", random_spd(131080, 10, 5, True), dict(fp32=True),
+          dict(precision="mixed"))]
+    # edges of the row ranges: 64-row tiles, 128 and 256 rows per workgroup,
+    # 1, 2, 4 logical workgroups per physical one, the block form's start
+    for n in (63, 64, 65, 127, 129, 4096, 4097, 16384, 16385, 32767, 32768, 65537, 131071):
+        c.append((f"rows_{n}", random_spd(n, 6, n), {}, {}))
+    c.append(("long_rows", random_spd(5000, 90, 7), {}, {}))
+    c.append(("long_rows_256", random_spd(40001, 60, 8), {}, {}))
+    for n in (131072, 131074, 200000, 262144, 262146):
+        c.append((f"blocks_{n}", random_spd(n, 8, n, True), {}, {}))
+    c.append(("long_blocks", random_spd(140002, 30, 9, True), {}, {}))
+    return c
+
+
+def digests():
+    capi.lib().nlInitExtension(b"HIP")
+    out = {}
+    for name, Sw, create, params in cases():
+        S = capi.System.from_crs(Sw, **create)
+        rows = []
+        for x0 in (None, np.linspace(-1.0, 1.0, Sw.n)):
+            x, st = S.solve(Sw.b, x0=x0, **params)
+            rows.append([hashlib.sha256(x.tobytes()).hexdigest(), st.iterations,
+                         st.outer_iterations, st.converged, st.extra_iterations,
+                         st.cg_rel_residual.hex(), st.rel_residual.hex()])
+        if "precision" not in params:  # the same solve in slices
+            S.solve_begin(Sw.b, **params)
+            for _ in range(2000):
+                fin, _ = S.solve_advance(3 if Sw.n < 5000 else 700)
+                if fin:
+                    break
+            x, st = S.solve_end()
+            rows.append([hashlib.sha256(x.tobytes()).hexdigest(), st.iterations])
+            assert rows[-1] == rows[0][:2], name
+        S.close()
+        out[name] = rows
+    return out
+
+
+def test_same_bits_as_three_launches(hip):
+    code = (f"import sys, json; sys.path[:0] = [{HERE!r}, {os.path.dirname(HERE)!r}]; "
+            "import test_gpu_cg_persist as t; print('DIGESTS' + json.dumps(t.digests()))")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100,
+                       env=dict(os.environ, NLHIP_DIRECT_LAUNCH="1"))
+    assert r.returncode == 0, r.stderr[-2000:]
+    ref = json.loads(r.stdout.split("DIGESTS")[1])
+    got = digests()
+    assert set(got) == set(ref)
+    for name in got:
+        assert got[name] == ref[name], name
