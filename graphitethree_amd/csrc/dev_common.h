@@ -76,6 +76,11 @@ __device__ __forceinline__ T group_sum(T v) {
     return v;
 }
 
+// Lane l's word in every lane (l uniform).
+__device__ __forceinline__ uint32_t lane_word(uint32_t v, int l) {
+    return uint32_t(__builtin_amdgcn_readlane(int(v), l));
+}
+
 // Block-wide sum; the result is returned to every thread.  `lds` must hold
 // kWavesPerBlock elements.  Deterministic: waves summed in index order.
 template <typename T>

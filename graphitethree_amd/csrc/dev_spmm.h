@@ -6,195 +6,211 @@
 
 namespace nlhip {
 
-constexpr uint32_t kSpmmChunk = 1024;  // (colind, val) entries staged in LDS at a time
-constexpr uint32_t kSpmmPass = 64;     // rows per pass (at least)
-constexpr int kSpmmU = 8;              // gathers in flight per lane
+constexpr int kSpmmU = 8;  // gathers in flight per lane
 
-// Rows of one pass of the engine for G lanes per row.
-template <int G>
-constexpr uint32_t spmm_pass_rows() {
-    return uint32_t(kBlock / G) > kSpmmPass ? uint32_t(kBlock / G) : kSpmmPass;
+// Rows of an XCD's blocks [lo, hi) of P: an even share of the m rows.
+__device__ __forceinline__ void spmm_xcd_rows(uint32_t m, uint32_t lo, uint32_t hi, uint32_t P,
+                                              uint32_t& r0, uint32_t& r1) {
+    r0 = uint32_t(uint64_t(m) * lo / P);
+    r1 = uint32_t(uint64_t(m) * hi / P);
 }
 
-// Rows of logical block L (the passes of max(64, kBlock / G) consecutive rows
-// of its XCD's range that fall to it in turn, see below): for each pass the
-// block copies the pass's (colind, val) range into LDS with coalesced
-// loads, then each G-lane group sums its rows of the pass from LDS, lane j
-// gathering X[col * k + j].  Row sums are left to right with one rounding
-// per product and per add.  For each row, lane j calls pre(row, j) (loads
-// the epilogue needs that do not depend on the sum) and then
-// fin(row, j, sum, pre value), row by row in the same order whatever the
-// path.  Every thread of the block must call this (it synchronises the
-// block).  zero_x: X is all zeros; the rows' sums are +0 (what the sums
-// would give) and the matrix is not read.
+// A lane's V adjacent columns of an interleaved vector (V = 2: an aligned
+// pair), loaded and stored as one word.  Stores are non-temporal: the result
+// must not push the gathered rows out of the L2.
+template <int V, typename T>
+struct Lane {
+    T v[V];
+};
+template <int V, typename T>
+__device__ __forceinline__ Lane<V, T> lane_load(const T* p) {
+    Lane<V, T> r;
+    __builtin_memcpy(r.v, p, sizeof(T) * V);
+    return r;
+}
+template <int V, typename T>
+__device__ __forceinline__ void lane_store(T* p, const T (&v)[V]) {
+    if constexpr (V == 2) {
+        using V2 = T __attribute__((ext_vector_type(2)));
+        V2 w;
+        w.x = v[0];
+        w.y = v[1];
+        __builtin_nontemporal_store(w, reinterpret_cast<V2*>(p));
+    } else {
+        __builtin_nontemporal_store(v[0], p);
+    }
+}
+
+// Row engine: G lanes per row (V = 1 or 2 adjacent columns each, gathered as
+// one copy per entry; G V >= k), 64 / G rows per wavefront and step.  The
+// blocks that run on one XCD share an even part of the rows and take its
+// steps in turn, so at any time they work on neighbouring rows and the X rows
+// that those gather (a stencil's rows i - w .. i + w) stay in that XCD's L2;
+// a wavefront's step is short (4 rows at 16 lanes), which keeps that window at
+// a megabyte for 256-byte X rows.
 //
-// ONE: every pass's entries fit in one LDS chunk (the caller checked it,
-// spmm_one_chunk): a group finishes each row before the next, holding
-// one accumulator and issuing the row's epilogue loads with its gathers.
-// Otherwise passes are staged in chunks and the group keeps one accumulator
-// per row of the pass until the pass ends.
-// V columns per lane (V = 1 or 2): lane j of a group owns columns
-// j*V .. j*V + V - 1, gathers them as one copy per entry (16 bytes for two
-// FP64 columns; k * V-aligned when V = 2 and k is even) and sums each of
-// them as above; pre / fin are called per column, columns in order.  G
-// lanes per row cover G * V >= k columns.
-template <int G, int V, bool ONE, typename T, typename Pre, typename Fin>
-__device__ __forceinline__ void spmm_rows_v(uint32_t m, uint32_t k, uint32_t rows_per_block,
-                                            uint32_t L, const uint32_t* __restrict__ rp,
+// A wavefront's rows are one contiguous range of entries: its lanes load them
+// coalesced, a step ahead, stage them in the wavefront's own LDS and each
+// row's lanes read them back (one address per row: a broadcast) for the
+// gathers of X[col * k + j].  No workgroup barrier: the wavefronts of a CU
+// drift apart and cover one another's latency.  The row pointers are loaded
+// two steps ahead, the next step's entries behind the first gathers (loads
+// return in order).
+//
+// Row sums are left to right with one rounding per product and per add.  For
+// each row, the lane with columns j .. j + V - 1 calls pre(row, j) (loads the
+// epilogue needs that do not depend on the sums) and then fin(row, j, sums,
+// pre value).  Columns with
+// done[j] set gather nothing (their sums are not used).  zero_x: X is all
+// zeros; the rows' sums are +0 (what the sums would give) and the matrix is
+// not read.
+//
+// Against the engine it replaces (passes of 64 rows staged by the whole
+// workgroup between barriers, and row shares rounded up to 64 rows per
+// block, which left most XCDs without rows below some 300 k rows):
+// the Chebyshev step at 90 k rows and 32 columns 37 -> 20 us, the SpMM of 2.25 M
+// rows and 32 columns 498 -> 428 us (1.12 GB fetched where 0.78 are needed,
+// 1.64 before; 471 us with plain stores; more wavefronts with fewer registers
+// spill: 445 us).  Grids are what is resident: with more workgroups the
+// waiting ones come back to rows that have left the L2 (550 us).
+template <int G, int V, typename T, typename Pre, typename Fin>
+__device__ __forceinline__ void spmm_rows_v(uint32_t m, uint32_t k, uint32_t L,
+                                            const uint32_t* __restrict__ rp,
                                             const uint32_t* __restrict__ ci,
                                             const T* __restrict__ val, const T* __restrict__ X,
                                             Pre& pre, Fin& fin, const int32_t* done = nullptr,
                                             bool zero_x = false) {
     static_assert(V == 1 || V == 2, "one or two columns per lane");
-    __shared__ uint32_t s_ci[kSpmmChunk];
-    __shared__ T s_val[kSpmmChunk];
-    constexpr uint32_t groups = kBlock / G;
-    constexpr uint32_t pass = spmm_pass_rows<G>();
-    const uint32_t g = threadIdx.x / G, jb = (threadIdx.x % G) * V;
+    constexpr uint32_t Rw = kWave / G;           // rows per wavefront and step
+    constexpr int C = G <= 8 ? 2 : 1;            // staged entries per lane
+    constexpr uint32_t kChunk = 64u * C;
+    __shared__ uint32_t s_ci[kWavesPerBlock][kChunk];
+    __shared__ T s_val[kWavesPerBlock][kChunk];
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint32_t w = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave)));
+    uint32_t* const sc = s_ci[w];
+    T* const sv = s_val[w];
+    const uint32_t g = lane / G, jb = (lane % G) * V;
     const bool mine = jb < k;  // the lane owns at least one column
-    // columns that have stopped gather nothing (their sums are not used)
     bool active_col = false;
 #pragma unroll
     for (int v = 0; v < V; ++v)
         active_col |= jb + v < k && !(done && done[jb + v]);
-    // the blocks that run on one XCD take the passes of their joint row range
-    // in turn, so at any time they work on neighbouring rows and the X rows
-    // those gather (a stencil's rows i - w .. i + w) are shared in that
-    // XCD's L2 instead of fetched once per block
-    uint32_t lo, hi;
+    uint32_t lo, hi, r0, r1;
     xcd_block_range(L, gridDim.x, lo, hi);
-    const uint64_t xb0 = uint64_t(lo) * rows_per_block, xb1 = uint64_t(hi) * rows_per_block;
-    const uint32_t r0 = xb0 < m ? uint32_t(xb0) : m;
-    const uint32_t r1 = xb1 < m ? uint32_t(xb1) : m;
-    const uint32_t first = uint32_t(uint64_t(L - lo) * pass);
-    const uint32_t step = (hi - lo) * pass;
-    constexpr uint32_t R = pass / groups;  // rows per group in one pass
-    // U gathers of entries [p, hi) (LDS offsets), added in order to acc
-    auto gather = [&](uint32_t p, uint32_t hi, T (&acc)[V]) {
-        T av[kSpmmU], xv[kSpmmU][V];
-#pragma unroll
-        for (int u = 0; u < kSpmmU; ++u) {
-            const uint32_t q = p + u < hi ? p + u : hi - 1u;
-            av[u] = s_val[q];
-            if (active_col) {
-                __builtin_memcpy(xv[u], X + uint64_t(s_ci[q]) * k + jb, sizeof(T) * V);
-            } else {
-#pragma unroll
-                for (int v = 0; v < V; ++v) xv[u][v] = T(0);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kSpmmU; ++u)
-            if (p + u < hi) {
-#pragma unroll
-                for (int v = 0; v < V; ++v) acc[v] = add_rn(acc[v], mul_rn(av[u], xv[u][v]));
-            }
-    };
+    spmm_xcd_rows(m, lo, hi, gridDim.x, r0, r1);
+    const uint64_t stride = uint64_t(hi - lo) * kWavesPerBlock * Rw;
+    uint64_t a = uint64_t(r0) + (uint64_t(L - lo) * kWavesPerBlock + w) * Rw;
     using PV = decltype(pre(0u, 0u));
-    auto finish = [&](uint32_t row, const T (&acc)[V], const PV (&pv)[V]) {
+    if (zero_x) {
+        for (; a < r1; a += stride) {
+            const uint64_t row = a + g;
+            if (row >= r1 || !mine) continue;
+            const PV pv = pre(uint32_t(row), jb);
+            T z[V];
 #pragma unroll
-        for (int v = 0; v < V; ++v)
-            if (jb + v < k) fin(row, jb + v, acc[v], pv[v]);
-    };
-    auto fetch = [&](uint32_t row, PV (&pv)[V]) {
-#pragma unroll
-        for (int v = 0; v < V; ++v)
-            if (jb + v < k) pv[v] = pre(row, jb + v);
-    };
-    for (uint64_t a64 = uint64_t(r0) + first; a64 < r1; a64 += step) {
-        const uint32_t a = uint32_t(a64);
-        const uint32_t pe = (a + pass < r1) ? a + pass : r1;
-        const uint32_t J0 = rp[a], J1 = rp[pe];
-        if (zero_x) {  // X = 0: every sum is +0 (block-uniform)
-            for (uint32_t t = 0; t < R; ++t) {
-                const uint32_t row = a + t * groups + g;
-                if (row >= pe) break;
-                if (!mine) continue;
-                PV pv[V]{};
-                fetch(row, pv);
-                T z[V];
-#pragma unroll
-                for (int v = 0; v < V; ++v) z[v] = T(0);
-                finish(row, z, pv);
-            }
-            continue;
+            for (int v = 0; v < V; ++v) z[v] = T(0);
+            fin(uint32_t(row), jb, z, pv);
         }
-        if constexpr (ONE) {
-            __syncthreads();  // the previous pass has been consumed
-            for (uint32_t q = J0 + threadIdx.x; q < J1; q += kBlock) {
-                s_ci[q - J0] = ci[q];
-                s_val[q - J0] = val[q];
-            }
-            __syncthreads();
-            for (uint32_t t = 0; t < R; ++t) {
-                const uint32_t row = a + t * groups + g;
-                if (row >= pe) break;
-                const uint32_t lo = rp[row] - J0, hi = rp[row + 1] - J0;
-                PV pv[V]{};
-                if (mine) fetch(row, pv);
-                T acc[V];
-#pragma unroll
-                for (int v = 0; v < V; ++v) acc[v] = T(0);
-                for (uint32_t p = lo; p < hi; p += kSpmmU) gather(p, hi, acc);
-                if (mine) finish(row, acc, pv);
-            }
-        } else {
-            uint32_t rb[R], re[R];
-            T acc[R][V];
-#pragma unroll
-            for (uint32_t t = 0; t < R; ++t) {
-                const uint32_t row = a + t * groups + g;
-                rb[t] = re[t] = 0;
-                if (row < pe) {
-                    rb[t] = rp[row];
-                    re[t] = rp[row + 1];
-                }
-#pragma unroll
-                for (int v = 0; v < V; ++v) acc[t][v] = T(0);
-            }
-            for (uint32_t c0 = J0; c0 < J1; c0 += kSpmmChunk) {
-                const uint32_t c1 = (c0 + kSpmmChunk < J1) ? c0 + kSpmmChunk : J1;
-                __syncthreads();  // the previous chunk has been consumed
-                for (uint32_t q = c0 + threadIdx.x; q < c1; q += kBlock) {
-                    s_ci[q - c0] = ci[q];
-                    s_val[q - c0] = val[q];
-                }
-                __syncthreads();
-#pragma unroll
-                for (uint32_t t = 0; t < R; ++t) {
-                    const uint32_t lo = rb[t] > c0 ? rb[t] : c0, hi = re[t] < c1 ? re[t] : c1;
-                    for (uint32_t p = lo; p < hi; p += kSpmmU) gather(p - c0, hi - c0, acc[t]);
-                }
-            }
-#pragma unroll
-            for (uint32_t t = 0; t < R; ++t) {
-                const uint32_t row = a + t * groups + g;
-                if (mine && row < pe) {
-                    PV pv[V]{};
-                    fetch(row, pv);
-                    finish(row, acc[t], pv);
-                }
-            }
-        }
+        return;
     }
-}
-
-// One column per lane (spmm_rows_v with V = 1): lane j of a group owns
-// column j.
-template <int G, bool ONE, typename T, typename Pre, typename Fin>
-__device__ __forceinline__ void spmm_rows(uint32_t m, uint32_t k, uint32_t rows_per_block,
-                                          uint32_t L, const uint32_t* __restrict__ rp,
-                                          const uint32_t* __restrict__ ci,
-                                          const T* __restrict__ val, const T* __restrict__ X,
-                                          Pre& pre, Fin& fin, const int32_t* done = nullptr,
-                                          bool zero_x = false) {
-    spmm_rows_v<G, 1, ONE>(m, k, rows_per_block, L, rp, ci, val, X, pre, fin, done, zero_x);
+    auto row_ptrs = [&](uint64_t at, uint32_t& b, uint32_t& e) {
+        const uint64_t row = at + g;
+        b = rp[row < r1 ? uint32_t(row) : r1];
+        e = rp[row + 1 < r1 ? uint32_t(row) + 1u : r1];
+    };
+    uint32_t cn[C] = {};
+    T vn[C] = {};
+    auto load = [&](uint32_t j0, uint32_t j1) {  // entries [j0, j0 + kChunk) up to j1
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const uint32_t j = j0 + uint32_t(c) * 64u + lane;
+            if (j < j1) {
+                cn[c] = ntload(ci + j);
+                vn[c] = ntload(val + j);
+            }
+        }
+    };
+    if (a >= r1) return;
+    uint32_t rb, re, rbn, ren;
+    row_ptrs(a, rb, re);
+    row_ptrs(a + stride, rbn, ren);
+    uint32_t J0 = lane_word(rb, 0), J1 = lane_word(re, kWave - 1);
+    load(J0, J1);
+    for (;;) {
+        const uint32_t row = uint32_t(a) + g;  // a + 64 < 2^32 unless past r1
+        const bool in = a + g < r1;
+        uint32_t rb2, re2;
+        row_ptrs(a + 2 * stride, rb2, re2);
+        PV pv{};
+        if (in && mine) pv = pre(row, jb);
+        T acc[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[v] = T(0);
+        const uint32_t K0 = lane_word(rbn, 0), K1 = lane_word(ren, kWave - 1);
+        for (uint32_t c0 = J0;; c0 += kChunk) {
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                sc[c * 64 + lane] = cn[c];
+                sv[c * 64 + lane] = vn[c];
+            }
+            __builtin_amdgcn_wave_barrier();
+            const bool last = c0 + kChunk >= J1 || c0 + kChunk < c0;
+            const uint32_t b = rb > c0 ? rb - c0 : 0u;
+            const uint32_t e = re > c0 ? (re - c0 < kChunk ? re - c0 : kChunk) : 0u;
+            // the next entries to load: the rest of this step's, or the next step's
+            const uint32_t n0 = last ? K0 : c0 + kChunk, n1 = last ? K1 : J1;
+            bool ahead = false;
+            for (uint32_t p = b; p < e || !ahead; p += kSpmmU) {
+                T xv[kSpmmU][V];
+                if (p < e) {
+#pragma unroll
+                    for (int u = 0; u < kSpmmU; ++u) {
+                        const uint32_t q = p + u < e ? p + u : e - 1u;
+                        if (active_col) {
+                            __builtin_memcpy(xv[u], X + uint64_t(sc[q]) * k + jb, sizeof(T) * V);
+                        } else {
+#pragma unroll
+                            for (int v = 0; v < V; ++v) xv[u][v] = T(0);
+                        }
+                    }
+                }
+                if (!ahead) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    load(n0, n1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    ahead = true;
+                }
+                if (p < e) {
+#pragma unroll
+                    for (int u = 0; u < kSpmmU; ++u)
+                        if (p + u < e) {
+                            const T av = sv[p + u];
+#pragma unroll
+                            for (int v = 0; v < V; ++v)
+                                acc[v] = add_rn(acc[v], mul_rn(av, xv[u][v]));
+                        }
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (last) break;
+        }
+        if (in && mine) fin(row, jb, acc, pv);
+        a += stride;
+        if (a >= r1) return;
+        rb = rbn;
+        re = ren;
+        rbn = rb2;
+        ren = re2;
+        J0 = K0;
+        J1 = K1;
+    }
 }
 
 // ---- stream SpMM for a few right-hand sides --------------------------
 //
-// For k <= 4 right-hand sides the row-group engine above leaves lanes idle
-// (4 lanes for k = 3) and waits for each pass's staging before it gathers.
+// For k <= 4 right-hand sides the row engine above leaves lanes idle (4 lanes
+// for k = 3).
 // This engine streams the matrix as the scalar stream engine does (one row
 // per lane, 64-row tiles, a wavefront's nonzeros as one contiguous range in
 // chunks of 64E entries, the next chunk's (colind, val) loads issued before

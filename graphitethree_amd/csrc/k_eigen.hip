@@ -18,26 +18,29 @@ namespace {
 constexpr uint32_t kGramTile = 64;  // rows per LDS tile of the Gram kernel
 
 // AY = A Y.
-template <int P, bool ONE>
-__global__ __launch_bounds__(kBlock) void k_eig_spmm(uint32_t n, uint32_t rpb, const uint32_t* rp,
+template <int P>
+__global__ __launch_bounds__(kBlock) void k_eig_spmm(uint32_t n, const uint32_t* rp,
                                                      const uint32_t* ci, const double* val,
                                                      const double* Y, double* AY) {
     const uint32_t L = xcd_logical_block(blockIdx.x, gridDim.x);
     auto pre = [](uint32_t, uint32_t) { return 0; };
-    auto fin = [&](uint32_t row, uint32_t j, double s, int) { AY[size_t(row) * P + j] = s; };
+    auto fin = [&](uint32_t row, uint32_t j, const double (&s)[2], int) {
+        lane_store<2>(AY + size_t(row) * P + j, s);
+    };
     // two columns per lane: P / 2 lanes per row, one 16-byte gather per entry
-    spmm_rows_v<P / 2, 2, ONE>(n, P, rpb, L, rp, ci, val, Y, pre, fin);
+    spmm_rows_v<P / 2, 2>(n, P, L, rp, ci, val, Y, pre, fin);
 }
 
 // One step of the Chebyshev recurrence on T = M^-1 A:
 //   Ynew = (T Y - c Y) s1 - s2 Xold       (s2 = 0 and no Xold on the first)
 // The row's minv, Y and Xold are loaded with its gathers.
 struct ChebPre {
-    double minv, y, xold;
+    double minv;
+    Lane<2, double> y, xold;
 };
 
-template <int P, bool ONE>
-__global__ __launch_bounds__(kBlock) void k_eig_cheb(uint32_t n, uint32_t rpb, const uint32_t* rp,
+template <int P>
+__global__ __launch_bounds__(kBlock) void k_eig_cheb(uint32_t n, const uint32_t* rp,
                                                      const uint32_t* ci, const double* val,
                                                      const double* minv, const double* Y,
                                                      const double* Xold, double* Ynew, double c,
@@ -45,16 +48,21 @@ __global__ __launch_bounds__(kBlock) void k_eig_cheb(uint32_t n, uint32_t rpb, c
     const uint32_t L = xcd_logical_block(blockIdx.x, gridDim.x);
     auto pre = [&](uint32_t row, uint32_t j) {
         const size_t i = size_t(row) * P + j;
-        return ChebPre{minv ? minv[row] : 1.0, Y[i], Xold ? Xold[i] : 0.0};
+        return ChebPre{minv ? minv[row] : 1.0, lane_load<2>(Y + i),
+                       Xold ? lane_load<2>(Xold + i) : Lane<2, double>{{0.0, 0.0}}};
     };
-    auto fin = [&](uint32_t row, uint32_t j, double s, const ChebPre& pv) {
-        const double t = minv ? mul_rn(s, pv.minv) : s;
-        double v = mul_rn(add_rn(t, -mul_rn(c, pv.y)), s1);
-        if (Xold) v = add_rn(v, -mul_rn(s2, pv.xold));
-        Ynew[size_t(row) * P + j] = v;
+    auto fin = [&](uint32_t row, uint32_t j, const double (&s)[2], const ChebPre& pv) {
+        double v[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const double t = minv ? mul_rn(s[q], pv.minv) : s[q];
+            v[q] = mul_rn(add_rn(t, -mul_rn(c, pv.y.v[q])), s1);
+            if (Xold) v[q] = add_rn(v[q], -mul_rn(s2, pv.xold.v[q]));
+        }
+        lane_store<2>(Ynew + size_t(row) * P + j, v);
     };
     // two columns per lane: P / 2 lanes per row, one 16-byte gather per entry
-    spmm_rows_v<P / 2, 2, ONE>(n, P, rpb, L, rp, ci, val, Y, pre, fin);
+    spmm_rows_v<P / 2, 2>(n, P, L, rp, ci, val, Y, pre, fin);
 }
 
 // Per workgroup b: part[b][i][j] = sum over its rows r (in order) of
@@ -264,40 +272,31 @@ uint32_t rows_per_group(uint32_t n) {
     }
 
 EigShape eig_shape(uint32_t n, uint32_t p, int cu) {
-    // G = p lanes per row, passes of 64 rows; at most 16 workgroups per CU
-    const uint32_t per = 256u / p;
-    const uint64_t passes = (uint64_t(n) + per - 1) / per;
-    const uint64_t cap = uint64_t(cu > 0 ? cu : 1) * 16;
+    // p / 2 lanes per row; at most as many workgroups as are resident, so that
+    // those of an XCD stay on neighbouring rows
+    const uint32_t per = kBlock / (p / 2);
+    const uint64_t steps = (uint64_t(n) + per - 1) / per;
+    int res = 0;
+    const void* f = nullptr;
+    NLHIP_EIG_P(p, (f = reinterpret_cast<const void*>(&k_eig_cheb<PP>)));
+    NLHIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&res, f, kBlock, 0));
+    const uint64_t cap = uint64_t(cu > 0 ? cu : 1) * uint64_t(res > 0 ? res : 1);
     EigShape e;
-    e.grid = uint32_t(passes < 1 ? 1 : (passes < cap ? passes : cap));
-    uint64_t rpb = (uint64_t(n) + e.grid - 1) / e.grid;
-    rpb = (rpb + kSpmmPass - 1) / kSpmmPass * kSpmmPass;
-    e.rows_per_block = uint32_t(rpb < kSpmmPass ? kSpmmPass : rpb);
+    e.grid = uint32_t(steps < 1 ? 1 : (steps < cap ? steps : cap));
     return e;
 }
 
 void eig_spmm(const EigShape& e, uint32_t n, uint32_t p, const uint32_t* rp, const uint32_t* ci,
               const double* val, const double* Y, double* AY, hipStream_t s) {
-    if (e.one_chunk) {
-        NLHIP_EIG_P(p, (k_eig_spmm<PP, true><<<e.grid, kBlock, 0, s>>>(n, e.rows_per_block, rp, ci,
-                                                                    val, Y, AY)));
-    } else {
-        NLHIP_EIG_P(p, (k_eig_spmm<PP, false><<<e.grid, kBlock, 0, s>>>(n, e.rows_per_block, rp,
-                                                                     ci, val, Y, AY)));
-    }
+    NLHIP_EIG_P(p, (k_eig_spmm<PP><<<e.grid, kBlock, 0, s>>>(n, rp, ci, val, Y, AY)));
     NLHIP_CHECK(hipGetLastError());
 }
 
 void eig_cheb(const EigShape& e, uint32_t n, uint32_t p, const uint32_t* rp, const uint32_t* ci,
               const double* val, const double* minv, const double* Y, const double* Xold,
               double* Ynew, double c, double s1, double s2, hipStream_t s) {
-    if (e.one_chunk) {
-        NLHIP_EIG_P(p, (k_eig_cheb<PP, true><<<e.grid, kBlock, 0, s>>>(
-                           n, e.rows_per_block, rp, ci, val, minv, Y, Xold, Ynew, c, s1, s2)));
-    } else {
-        NLHIP_EIG_P(p, (k_eig_cheb<PP, false><<<e.grid, kBlock, 0, s>>>(
-                           n, e.rows_per_block, rp, ci, val, minv, Y, Xold, Ynew, c, s1, s2)));
-    }
+    NLHIP_EIG_P(p, (k_eig_cheb<PP><<<e.grid, kBlock, 0, s>>>(n, rp, ci, val, minv, Y, Xold, Ynew,
+                                                             c, s1, s2)));
     NLHIP_CHECK(hipGetLastError());
 }
 

@@ -11,8 +11,8 @@
 // * k <= kMultiStreamMaxK: the stream engine, one row per lane, the matrix
 //   streamed in 64-row tiles and each entry's k values gathered as one copy;
 //   Pdq workgroups of sp tiles, as many as the device holds at once;
-// * larger k: G-lane row groups (G = k rounded up to a power of two, lane j
-//   owning right-hand side j), (val, colind) staged in LDS once per pass.
+// * larger k: the row engine, G lanes per row (G = k rounded up to a power of
+//   two, or half of it with two columns per lane).
 //
 // Per iteration, 5 launches: direction D = beta_j D + H; SpMM Q = A D with
 // per-workgroup partials of d_j.q_j; a reduction launch (alpha_j); update
@@ -29,7 +29,7 @@
 namespace nlhip {
 
 // Rows [r0, r1) of logical block L for the element-wise kernels, with the
-// same G-lane groups as spmm_rows: thread t handles column t % G of rows
+// G-lane row groups: thread t handles column t % G of rows
 // r0 + t / G, r0 + t / G + kBlock / G, ...
 __device__ __forceinline__ void block_rows(const uint32_t m, const uint32_t rows_per_block,
                                            uint32_t L, uint32_t& r0, uint32_t& r1) {
@@ -92,7 +92,7 @@ constexpr int two_cols_v() {
     return G >= 8 ? 2 : 1;
 }
 
-template <int G, int V, bool ONE, typename T, bool PREC>
+template <int G, int V, typename T, bool PREC>
 __global__ __launch_bounds__(kBlock) void k_m_init(MultiArgs<T> a) {
     __shared__ T lds[kBlock * V];
     const uint32_t L = xcd_logical_block(blockIdx.x, gridDim.x);
@@ -100,23 +100,29 @@ __global__ __launch_bounds__(kBlock) void k_m_init(MultiArgs<T> a) {
     T prh[V], prr[V], pbb[V];
 #pragma unroll
     for (int c = 0; c < V; ++c) prh[c] = prr[c] = pbb[c] = T(0);
-    auto pre = [&](uint32_t row, uint32_t j) {
-        return Pair<T>{a.b[uint64_t(row) * k + j], PREC ? a.dinv[row] : T(1)};
+    struct PV {
+        Lane<V, T> b;
+        T dinv;
     };
-    auto fin = [&](uint32_t row, uint32_t j, T s, const Pair<T>& pv) {
-        const uint64_t i = uint64_t(row) * k + j;
-        const T bi = pv.a;
-        const T ri = add_rn(s, mul_rn(T(-1), bi));
-        const T hi = PREC ? mul_rn(pv.b, ri) : ri;
-        a.r[i] = ri;
-        a.h[i] = hi;
-        const uint32_t c = j % V;  // the lane's columns are j - c .. j - c + V - 1
-        prh[c] += ri * hi;
-        prr[c] += ri * ri;
-        pbb[c] += bi * bi;
+    auto pre = [&](uint32_t row, uint32_t j) {
+        return PV{lane_load<V>(a.b + uint64_t(row) * k + j), PREC ? a.dinv[row] : T(1)};
+    };
+    auto fin = [&](uint32_t row, uint32_t j, const T (&s)[V], const PV& pv) {
+        T r[V], h[V];
+#pragma unroll
+        for (int c = 0; c < V; ++c) {
+            const T bi = pv.b.v[c];
+            r[c] = add_rn(s[c], mul_rn(T(-1), bi));
+            h[c] = PREC ? mul_rn(pv.dinv, r[c]) : r[c];
+            prh[c] += r[c] * h[c];
+            prr[c] += r[c] * r[c];
+            pbb[c] += bi * bi;
+        }
+        lane_store<V>(a.r + uint64_t(row) * k + j, r);
+        lane_store<V>(a.h + uint64_t(row) * k + j, h);
     };
     const bool zero_x = a.x_nonzero && *a.x_nonzero == 0;  // X = 0: A X = 0 (block-uniform)
-    spmm_rows_v<G / V, V, ONE>(a.m, k, a.rows_per_block, L, a.rp, a.ci, a.val, a.x, pre, fin,
+    spmm_rows_v<G / V, V>(a.m, k, L, a.rp, a.ci, a.val, a.x, pre, fin,
                                nullptr, zero_x);
     column_partials_v<V>(prh, k, G / V, lds, a.part_rh + size_t(L) * k);
     column_partials_v<V>(prr, k, G / V, lds, a.part_rr + size_t(L) * k);
@@ -186,7 +192,7 @@ __global__ __launch_bounds__(kBlock) void k_m_dir(MultiArgs<T> a) {
     }
 }
 
-template <int G, int V, bool ONE, typename T>
+template <int G, int V, typename T>
 __global__ __launch_bounds__(kBlock) void k_m_spmm(MultiArgs<T> a) {
     __shared__ T lds[kBlock * V];
     if (!any_active(a)) return;  // every column has stopped (block-uniform)
@@ -195,12 +201,15 @@ __global__ __launch_bounds__(kBlock) void k_m_spmm(MultiArgs<T> a) {
     T pdq[V];
 #pragma unroll
     for (int c = 0; c < V; ++c) pdq[c] = T(0);
-    auto pre = [&](uint32_t row, uint32_t j) { return a.d[uint64_t(row) * k + j]; };
-    auto fin = [&](uint32_t row, uint32_t j, T s, T di) {
-        a.q[uint64_t(row) * k + j] = s;
-        pdq[j % V] += di * s;
+    auto pre = [&](uint32_t row, uint32_t j) {
+        return lane_load<V>(a.d + uint64_t(row) * k + j);
     };
-    spmm_rows_v<G / V, V, ONE>(a.m, k, a.rows_per_block, L, a.rp, a.ci, a.val, a.d, pre, fin,
+    auto fin = [&](uint32_t row, uint32_t j, const T (&s)[V], const Lane<V, T>& d) {
+        lane_store<V>(a.q + uint64_t(row) * k + j, s);
+#pragma unroll
+        for (int c = 0; c < V; ++c) pdq[c] += d.v[c] * s[c];
+    };
+    spmm_rows_v<G / V, V>(a.m, k, L, a.rp, a.ci, a.val, a.d, pre, fin,
                                a.done);
     column_partials_v<V>(pdq, k, G / V, lds, a.part_dq + size_t(L) * k);
 }
@@ -442,7 +451,7 @@ __global__ __launch_bounds__(kBlock) void k_to_colmajor(uint32_t n, uint32_t k, 
 }
 
 // R = B - A X (FP64, interleaved), per-column partial |r|^2 and |b|^2.
-template <int G, int V, bool ONE>
+template <int G, int V>
 __global__ __launch_bounds__(kBlock) void k_m_residual64(MultiArgs<double> a) {
     __shared__ double lds[kBlock * V];
     const uint32_t L = xcd_logical_block(blockIdx.x, gridDim.x);
@@ -450,14 +459,20 @@ __global__ __launch_bounds__(kBlock) void k_m_residual64(MultiArgs<double> a) {
     double prr[V], pbb[V];
 #pragma unroll
     for (int c = 0; c < V; ++c) prr[c] = pbb[c] = 0.0;
-    auto pre = [&](uint32_t row, uint32_t j) { return a.b[uint64_t(row) * k + j]; };
-    auto fin = [&](uint32_t row, uint32_t j, double s, double bi) {
-        const double ri = bi - s;
-        a.r[uint64_t(row) * k + j] = ri;
-        prr[j % V] += ri * ri;
-        pbb[j % V] += bi * bi;
+    auto pre = [&](uint32_t row, uint32_t j) {
+        return lane_load<V>(a.b + uint64_t(row) * k + j);
     };
-    spmm_rows_v<G / V, V, ONE>(a.m, k, a.rows_per_block, L, a.rp, a.ci, a.val, a.x, pre, fin);
+    auto fin = [&](uint32_t row, uint32_t j, const double (&s)[V], const Lane<V, double>& b) {
+        double r[V];
+#pragma unroll
+        for (int c = 0; c < V; ++c) {
+            r[c] = b.v[c] - s[c];
+            prr[c] += r[c] * r[c];
+            pbb[c] += b.v[c] * b.v[c];
+        }
+        lane_store<V>(a.r + uint64_t(row) * k + j, r);
+    };
+    spmm_rows_v<G / V, V>(a.m, k, L, a.rp, a.ci, a.val, a.x, pre, fin);
     column_partials_v<V>(prr, k, G / V, lds, a.part_rr + size_t(L) * k);
     column_partials_v<V>(pbb, k, G / V, lds, a.part_bb + size_t(L) * k);
 }
@@ -557,10 +572,7 @@ __global__ __launch_bounds__(kBlock) void k_m_ir_update(MultiArgs<double> a64,
 // ------------------------------------------------------------- launchers
 
 #define NLHIP_G_SWITCH(G_, CALL)                         \
-    switch (G_) {                                        \
-        case 1: { constexpr int G = 1; CALL; } break;    \
-        case 2: { constexpr int G = 2; CALL; } break;    \
-        case 4: { constexpr int G = 4; CALL; } break;    \
+    switch (G_) { /* k > kMultiStreamMaxK */             \
         case 8: { constexpr int G = 8; CALL; } break;    \
         case 16: { constexpr int G = 16; CALL; } break;  \
         case 32: { constexpr int G = 32; CALL; } break;  \
@@ -588,44 +600,32 @@ static uint32_t ew_grid_m(uint64_t n) {
 }
 
 namespace {
-
-__global__ void k_window_max(uint32_t m, const uint32_t* rp, uint32_t pass, uint32_t* out) {
-    const uint32_t nw = (m + 7) / 8;
-    const uint32_t stride = gridDim.x * blockDim.x;
-    uint32_t best = 0;
-    for (uint32_t w = blockIdx.x * blockDim.x + threadIdx.x; w < nw; w += stride) {
-        const uint32_t a = 8 * w;
-        const uint32_t e = (uint64_t(a) + pass < m) ? a + pass : m;
-        const uint32_t c = rp[e] - rp[a];
-        best = c > best ? c : best;
-    }
-    atomicMax(out, best);
-}
-
-}  // namespace
-
-// The largest number of entries in `pass` consecutive rows starting at a
-// multiple of 8 rows: every pass spmm_rows takes starts at such a row
-// (blocks hold multiples of 8 rows for every G).
-bool spmm_one_chunk(uint32_t m, const uint32_t* rp, uint32_t G, hipStream_t s) {
-    const uint32_t pass = std::max<uint32_t>(kBlock / G, kSpmmPass);
-    DevBuf<uint32_t> out(1);
-    NLHIP_CHECK(hipMemsetAsync(out.get(), 0, 4, s));
-    k_window_max<<<ew_grid_m((uint64_t(m) + 7) / 8), kBlock, 0, s>>>(m, rp, pass, out.get());
-    NLHIP_CHECK(hipGetLastError());
-    uint32_t h = 0;
-    NLHIP_CHECK(hipMemcpyAsync(&h, out.get(), 4, hipMemcpyDeviceToHost, s));
-    NLHIP_CHECK(hipStreamSynchronize(s));
-    return h <= kSpmmChunk;
-}
-
-namespace {
 template <typename T>
 hipError_t stream_spmm_kernel(uint32_t k, bool d16, const void*& f) {
     NLHIP_KD_SWITCH(k, d16, (f = reinterpret_cast<const void*>(&k_m_spmm_stream<K, D16, T>)));
     return hipSuccess;
 }
 }  // namespace
+
+template <typename T>
+uint32_t multi_rows_per_cu(uint32_t k) {
+    uint32_t G = 8;
+    while (G < k) G <<= 1;
+    const bool v2 = multi_two_cols<T>(k);
+    const void* f = nullptr;
+    auto pick = [&] {
+        NLHIP_G_SWITCH(G, (f = v2 ? reinterpret_cast<const void*>(&k_m_spmm<G, two_cols_v<G>(), T>)
+                                  : reinterpret_cast<const void*>(&k_m_spmm<G, 1, T>)));
+        return hipSuccess;
+    };
+    int per = 0;
+    if (pick() != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, f, kBlock, 0) != hipSuccess || per < 1)
+        return 1;
+    return uint32_t(per);
+}
+template uint32_t multi_rows_per_cu<double>(uint32_t);
+template uint32_t multi_rows_per_cu<float>(uint32_t);
 
 // Sized for the SpMM step, the launch of every iteration; the start and the
 // residual (once per solve, more registers for their epilogues at large k)
@@ -650,18 +650,12 @@ hipError_t multi_start(const MultiArgs<T>& a, bool precond, T eps, int max_iter,
         NLHIP_KD_SWITCH(a.k, d16, (k_m_init_stream<K, D16, T, true><<<a.Pdq, kBlock, 0, s>>>(a)));
     } else if (a.sp) {
         NLHIP_KD_SWITCH(a.k, d16, (k_m_init_stream<K, D16, T, false><<<a.Pdq, kBlock, 0, s>>>(a)));
-    } else if (precond && a.one_chunk) {
-        NLHIP_G_SWITCH(a.G, (v2 ? k_m_init<G, two_cols_v<G>(), true, T, true><<<a.P, kBlock, 0, s>>>(a)
-                               : k_m_init<G, 1, true, T, true><<<a.P, kBlock, 0, s>>>(a)));
     } else if (precond) {
-        NLHIP_G_SWITCH(a.G, (v2 ? k_m_init<G, two_cols_v<G>(), false, T, true><<<a.P, kBlock, 0, s>>>(a)
-                               : k_m_init<G, 1, false, T, true><<<a.P, kBlock, 0, s>>>(a)));
-    } else if (a.one_chunk) {
-        NLHIP_G_SWITCH(a.G, (v2 ? k_m_init<G, two_cols_v<G>(), true, T, false><<<a.P, kBlock, 0, s>>>(a)
-                               : k_m_init<G, 1, true, T, false><<<a.P, kBlock, 0, s>>>(a)));
+        NLHIP_G_SWITCH(a.G, (v2 ? k_m_init<G, two_cols_v<G>(), T, true><<<a.P, kBlock, 0, s>>>(a)
+                               : k_m_init<G, 1, T, true><<<a.P, kBlock, 0, s>>>(a)));
     } else {
-        NLHIP_G_SWITCH(a.G, (v2 ? k_m_init<G, two_cols_v<G>(), false, T, false><<<a.P, kBlock, 0, s>>>(a)
-                               : k_m_init<G, 1, false, T, false><<<a.P, kBlock, 0, s>>>(a)));
+        NLHIP_G_SWITCH(a.G, (v2 ? k_m_init<G, two_cols_v<G>(), T, false><<<a.P, kBlock, 0, s>>>(a)
+                               : k_m_init<G, 1, T, false><<<a.P, kBlock, 0, s>>>(a)));
     }
     k_m_sys_init<T><<<a.k, kBlock, 0, s>>>(a, eps, max_iter);
     return hipGetLastError();
@@ -675,12 +669,9 @@ hipError_t multi_iteration(const MultiArgs<T>& a, bool precond, int max_iter, hi
     if (a.sp) {
         NLHIP_KD_SWITCH(a.k, a.cols.ci16 != nullptr,
                         (k_m_spmm_stream<K, D16, T><<<a.Pdq, kBlock, 0, s>>>(a)));
-    } else if (a.one_chunk) {
-        NLHIP_G_SWITCH(a.G, (v2 ? k_m_spmm<G, two_cols_v<G>(), true, T><<<a.P, kBlock, 0, s>>>(a)
-                               : k_m_spmm<G, 1, true, T><<<a.P, kBlock, 0, s>>>(a)));
     } else {
-        NLHIP_G_SWITCH(a.G, (v2 ? k_m_spmm<G, two_cols_v<G>(), false, T><<<a.P, kBlock, 0, s>>>(a)
-                               : k_m_spmm<G, 1, false, T><<<a.P, kBlock, 0, s>>>(a)));
+        NLHIP_G_SWITCH(a.G, (v2 ? k_m_spmm<G, two_cols_v<G>(), T><<<a.P, kBlock, 0, s>>>(a)
+                               : k_m_spmm<G, 1, T><<<a.P, kBlock, 0, s>>>(a)));
     }
     k_m_reduce_alpha<T><<<cg, kBlock, 0, s>>>(a);
     if (precond) k_m_update<T, true><<<a.P, kBlock, 0, s>>>(a);
@@ -711,12 +702,9 @@ hipError_t multi_residual64(const MultiArgs<double>& a, hipStream_t s) {
     if (a.sp) {
         NLHIP_KD_SWITCH(a.k, a.cols.ci16 != nullptr,
                         (k_m_residual64_stream<K, D16><<<a.Pdq, kBlock, 0, s>>>(a)));
-    } else if (a.one_chunk) {
-        NLHIP_G_SWITCH(a.G, (v2 ? k_m_residual64<G, two_cols_v<G>(), true><<<a.P, kBlock, 0, s>>>(a)
-                               : k_m_residual64<G, 1, true><<<a.P, kBlock, 0, s>>>(a)));
     } else {
-        NLHIP_G_SWITCH(a.G, (v2 ? k_m_residual64<G, two_cols_v<G>(), false><<<a.P, kBlock, 0, s>>>(a)
-                               : k_m_residual64<G, 1, false><<<a.P, kBlock, 0, s>>>(a)));
+        NLHIP_G_SWITCH(a.G, (v2 ? k_m_residual64<G, two_cols_v<G>()><<<a.P, kBlock, 0, s>>>(a)
+                               : k_m_residual64<G, 1><<<a.P, kBlock, 0, s>>>(a)));
     }
     k_m_norms64<<<a.k, kBlock, 0, s>>>(a);
     return hipGetLastError();

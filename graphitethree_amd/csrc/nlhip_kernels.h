@@ -309,7 +309,6 @@ struct MultiArgs {
     uint32_t G;               // lanes per row: k rounded up to a power of two
     uint32_t P;               // workgroups of the row-shaped launches
     uint32_t rows_per_block;
-    uint32_t one_chunk;       // every SpMM pass fits one LDS chunk (spmm_window_max)
     const uint32_t* rp;
     const uint32_t* ci;
     const T* val;
@@ -352,6 +351,9 @@ constexpr uint32_t kMultiStreamMaxK = 4;
 // offsets or not) that one CU holds at once.
 template <typename T>
 uint32_t multi_stream_per_cu(uint32_t k, bool d16);
+// The same of the row engine's SpMM step (k > kMultiStreamMaxK).
+template <typename T>
+uint32_t multi_rows_per_cu(uint32_t k);
 
 template <typename T>
 hipError_t multi_start(const MultiArgs<T>& a, bool precond, T eps, int max_iter, hipStream_t s);

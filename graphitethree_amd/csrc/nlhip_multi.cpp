@@ -22,18 +22,22 @@ uint32_t pow2_ceil(uint32_t k) {
 }
 
 // Workgroups of the multi right-hand-side launches: enough for one pass of
-// G-lane row groups over the matrix, at most 16 per CU (the kernels use few
-// registers, so the extra waves hide the gather latency).
+// G-lane row groups over the matrix; at most 16 per CU when the SpMM step
+// streams (it has its own count), otherwise as many as the row engine's SpMM
+// step keeps resident (its workgroups take neighbouring rows in turn, so the
+// ones that wait for a place would come back to rows that have left the L2).
+template <typename T>
 uint32_t multi_grid(const System& S, uint32_t k) {
     const uint32_t per = 256u / pow2_ceil(k);
     const uint64_t passes = (uint64_t(S.n) + per - 1) / per;
-    const uint64_t cap = uint64_t(std::max(1, device().cu_count)) * 16;
+    const uint64_t cap = uint64_t(std::max(1, device().cu_count)) *
+                         (k <= kMultiStreamMaxK ? 16u : multi_rows_per_cu<T>(k));
     return uint32_t(std::max<uint64_t>(1, std::min(passes, cap)));
 }
 
 template <typename T>
 void multi_alloc(System& S, MultiWork<T>& w, uint32_t k) {
-    const uint32_t P = multi_grid(S, k);
+    const uint32_t P = multi_grid<T>(S, k);
     if (w.n == S.n && w.k == k && w.P == P && w.x.get()) return;
     w.graph.reset();
     w.n = S.n;
@@ -69,7 +73,6 @@ void multi_alloc(System& S, MultiWork<T>& w, uint32_t k) {
     uint64_t rpb = (uint64_t(S.n) + P - 1) / P;
     rpb = (rpb + rows_per_pass - 1) / rows_per_pass * rows_per_pass;
     a.rows_per_block = uint32_t(std::max<uint64_t>(rpb, rows_per_pass));
-    a.one_chunk = spmm_one_chunk(S.n, S.rowptr.get(), a.G, S.stream.get()) ? 1u : 0u;
     a.rp = S.rowptr.get();
     a.ci = S.colind.get();
     a.cols = S.cols();

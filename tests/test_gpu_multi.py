@@ -224,3 +224,29 @@ def test_context_nb_systems(hip):
     for j in range(3):
         xr, _, _ = O.pcg(A, Sw.rhs[j], eps=1e-12, max_iter=1000)
         assert rel(got[j], xr) <= REL_DIFF
+
+
+@pytest.mark.parametrize("k", [5, 6, 8, 10, 16, 18, 31, 32])
+@pytest.mark.parametrize("n,deg", [(1, 0), (2, 1), (15, 4), (257, 20), (2111, 200)])
+def test_row_engine_edges(hip, k, n, deg):
+    """k > 4 (4 to 32 lanes per row, one or two columns each): fewer rows
+    than lanes, a wavefront's step cut off by the end, empty and long rows
+    (more entries than a wavefront stages), against a dense product: the
+    residual of a solve with no iterations is B - A X0."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(1000 * k + n)
+    M = sp.random(n, n, density=min(1.0, deg / n), random_state=n, format="lil")
+    M[rng.integers(0, n)] = 0.0
+    M[rng.integers(0, n)] = rng.standard_normal(n)
+    M = M.tocsr()
+    M.sort_indices()
+    S = capi.System(M.indptr.astype(np.uint32), M.indices.astype(np.uint32), M.data)
+    X0, B = rng.standard_normal((k, n)), rng.standard_normal((k, n))
+    X, per, _ = S.solve_multi(B, X0=X0, max_iter=0, precond="none")
+    assert np.array_equal(X, X0)
+    for j in range(k):
+        want = np.linalg.norm(B[j] - M @ X0[j]) / np.linalg.norm(B[j])
+        # a row of L entries: (L + 2) roundings of terms of at most |A| |x|
+        tol = (n + 4) * 2.0 ** -52 * np.linalg.norm(abs(M) @ abs(X0[j]) + abs(B[j]))
+        assert abs(per[j].rel_residual - want) <= tol / np.linalg.norm(B[j]) + 1e-15 * want
+    S.close()
