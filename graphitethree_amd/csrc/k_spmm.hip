@@ -14,11 +14,22 @@
 // * larger k: the row engine, G lanes per row (G = k rounded up to a power of
 //   two, or half of it with two columns per lane).
 //
-// Per iteration, 5 launches: direction D = beta_j D + H; SpMM Q = A D with
-// per-workgroup partials of d_j.q_j; a reduction launch (alpha_j); update
-// X, R, H with partials of r_j.h_j and r_j.r_j; a reduction launch
-// (stopping test, beta_j).  Columns whose stopping test held are left
-// untouched; once every column has stopped, the launches exit at once.
+// An iteration is the single-right-hand-side one (k_cg.hip): direction
+// (x -= alpha d with the pending alpha, stopping test, d = beta d + h), SpMM
+// (Q = A D, partials of d_j.q_j), update (r -= alpha q, partials of r_j.h_j
+// and r_j.r_j).  h = D^-1 r is formed where it is read, from r and the one
+// D^-1 of the row, and not stored: 80 n k bytes per iteration with the SpMM's
+// 16, against 96 with h in memory and x updated beside r.
+// * k <= kMultiStreamMaxK: three launches, whose workgroups reduce the
+//   partials themselves (P k of them each);
+// * larger k: the scalars in launches of one workgroup per column in between
+//   (5 launches), where P k partials per workgroup would outweigh the step.
+// Against five launches each with h stored, us per iteration: 1500^2 rows,
+// k = 32, FP64 1700 -> 1350; 300^2, k = 3, FP64 25 -> 17 of kernel time; 1000^2,
+// k = 3, FP32 57 -> 41.
+// Columns whose stopping test held are left untouched (stop, raised with the
+// test, becomes done in the SpMM); once every column has stopped, the
+// launches exit at once.
 #include <algorithm>
 
 #include "dev_common.h"
@@ -38,43 +49,47 @@ __device__ __forceinline__ void block_rows(const uint32_t m, const uint32_t rows
     r1 = (uint64_t(r0) + rows_per_block < m) ? r0 + rows_per_block : m;
 }
 
-// Whether any column still iterates (its done flag, written by an earlier
-// launch, is clear); the same answer in every thread.
+// Whether any column's flags, written by earlier launches, are clear; the
+// same answer in every thread.  The direction step runs for columns that stop
+// in this iteration too (the pending update of x), the others do not.
 template <typename T>
-__device__ __forceinline__ bool any_active(const MultiArgs<T>& a) {
+__device__ __forceinline__ bool any_open(const MultiArgs<T>& a) {
     for (uint32_t j = 0; j < a.k; ++j)
         if (!a.done[j]) return true;
     return false;
 }
-
-// Per-workgroup partial sums of k columns: lds[kBlock] scratch; the group
-// lanes holding column j combine through LDS in a fixed order.
 template <typename T>
-__device__ __forceinline__ void column_partials(T v, uint32_t k, uint32_t G, T* lds,
-                                                T* out /* k values */) {
-    __syncthreads();
-    lds[threadIdx.x] = v;
-    __syncthreads();
-    if (threadIdx.x < k) {
-        T s = T(0);
-        for (uint32_t t = threadIdx.x; t < kBlock; t += G) s += lds[t];
-        out[threadIdx.x] = s;
-    }
+__device__ __forceinline__ bool any_active(const MultiArgs<T>& a) {
+    for (uint32_t j = 0; j < a.k; ++j)
+        if (!a.done[j] && !a.stop[j]) return true;
+    return false;
+}
+// In the SpMM launch, by one workgroup: columns that stopped in this
+// iteration are done (the direction launch has updated their x).  Workgroups
+// that read done[j] in this launch see stop[j] either way.
+template <typename T>
+__device__ __forceinline__ void close_stopped(const MultiArgs<T>& a) {
+    if (blockIdx.x == 0 && threadIdx.x < a.k && a.stop[threadIdx.x]) a.done[threadIdx.x] = 1;
 }
 
-// The same for V columns per lane (lane l of a G-lane row group holds the
-// partials of columns l*V .. l*V + V - 1); lds holds kBlock * V values.
+// Per-workgroup partial sums of k columns, V per lane (lane l of the lanes of
+// a row holds columns l*V .. l*V + V - 1): the lanes holding column j combine
+// through LDS in a fixed order; lds holds kBlock * V values.  The partials of
+// columns with done[j] or stop[j] set (may be null) stay as they are: a
+// re-opened column continues from them.
 template <int V, typename T>
-__device__ __forceinline__ void column_partials_v(const T (&v)[V], uint32_t k, uint32_t G,
-                                                  T* lds, T* out /* k values */) {
+__device__ __forceinline__ void column_partials_v(const T (&v)[V], uint32_t k, uint32_t lanes,
+                                                  T* lds, T* out /* k values */,
+                                                  const int32_t* done = nullptr,
+                                                  const int32_t* stop = nullptr) {
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < V; ++c) lds[threadIdx.x * V + c] = v[c];
     __syncthreads();
-    if (threadIdx.x < k) {
+    if (threadIdx.x < k && !(done && (done[threadIdx.x] || stop[threadIdx.x]))) {
         const uint32_t lane = threadIdx.x / V, c = threadIdx.x % V;
         T s = T(0);
-        for (uint32_t t = lane; t < kBlock; t += G) s += lds[t * V + c];
+        for (uint32_t t = lane; t < kBlock; t += lanes) s += lds[t * V + c];
         out[threadIdx.x] = s;
     }
 }
@@ -108,18 +123,17 @@ __global__ __launch_bounds__(kBlock) void k_m_init(MultiArgs<T> a) {
         return PV{lane_load<V>(a.b + uint64_t(row) * k + j), PREC ? a.dinv[row] : T(1)};
     };
     auto fin = [&](uint32_t row, uint32_t j, const T (&s)[V], const PV& pv) {
-        T r[V], h[V];
+        T r[V];
 #pragma unroll
         for (int c = 0; c < V; ++c) {
             const T bi = pv.b.v[c];
             r[c] = add_rn(s[c], mul_rn(T(-1), bi));
-            h[c] = PREC ? mul_rn(pv.dinv, r[c]) : r[c];
-            prh[c] += r[c] * h[c];
+            const T hi = PREC ? mul_rn(pv.dinv, r[c]) : r[c];
+            prh[c] += r[c] * hi;
             prr[c] += r[c] * r[c];
             pbb[c] += bi * bi;
         }
         lane_store<V>(a.r + uint64_t(row) * k + j, r);
-        lane_store<V>(a.h + uint64_t(row) * k + j, h);
     };
     const bool zero_x = a.x_nonzero && *a.x_nonzero == 0;  // X = 0: A X = 0 (block-uniform)
     spmm_rows_v<G / V, V>(a.m, k, L, a.rp, a.ci, a.val, a.x, pre, fin,
@@ -160,34 +174,188 @@ __global__ __launch_bounds__(kBlock) void k_m_sys_init(MultiArgs<T> a, T eps, in
         a.bb[j] = bb;
         a.thresh[j] = thresh;
         a.rho[j] = rho;
+        a.rho_prev[j] = T(1);
         a.err[j] = err;
         a.beta[j] = T(0);
         a.alpha[j] = T(0);
         a.iters[j] = 0;
+        a.stop[j] = 0;
         const bool skip = a.skip && a.skip[j];
         a.done[j] = (skip || !(err > thresh) || max_iter <= 0) ? 1 : 0;
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_m_dir(MultiArgs<T> a) {
-    if (!any_active(a)) return;  // every column has stopped
+// The sums of N x K interleaved partials (part[c][p K + j], p < P) over the
+// workgroups, in col_sum's order, in every thread; lds holds
+// kWavesPerBlock * N * K values.
+template <int N, int K, typename T>
+__device__ __forceinline__ void all_col_sums(const T* const (&part)[N], uint32_t P, T* lds,
+                                             T (&out)[N][K]) {
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+#pragma unroll
+    for (int c = 0; c < N; ++c)
+#pragma unroll
+        for (int j = 0; j < K; ++j) out[c][j] = T(0);
+    for (uint32_t p = threadIdx.x; p < P; p += kBlock)
+#pragma unroll
+        for (int c = 0; c < N; ++c)
+#pragma unroll
+            for (int j = 0; j < K; ++j) out[c][j] += part[c][size_t(p) * K + j];
+#pragma unroll
+    for (int c = 0; c < N; ++c)
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            const T v = group_sum<kWave>(out[c][j]);
+            if (lane == 0) lds[(c * K + j) * kWavesPerBlock + w] = v;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < N; ++c)
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            const T* l = lds + (c * K + j) * kWavesPerBlock;
+            out[c][j] = ((l[0] + l[1]) + l[2]) + l[3];
+        }
+}
+
+// Direction step for K <= kMultiStreamMaxK columns, one row per lane: the
+// scalars of every column from the last update's partials (block 0 writes
+// them), then x and d.
+template <int K, typename T, bool PREC>
+__global__ __launch_bounds__(kBlock) void k_m_dir_few(MultiArgs<T> a, int max_iter) {
+    __shared__ T lds[kWavesPerBlock * 2 * K];
+    if (!any_open(a)) return;  // every column has stopped
+    T sums[2][K];
+    const T* const parts[2] = {a.part_rh, a.part_rr};
+    all_col_sums<2, K>(parts, a.P, lds, sums);
+    bool upd[K], dir[K], first[K];
+    T alpha[K], beta[K];
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        const int it = a.iters[j];
+        const bool open = !a.done[j];
+        first[j] = it == 0;  // its scalars and test: the start's
+        const bool stop = !first[j] && (!(sums[1][j] > a.thresh[j]) || it >= max_iter);
+        alpha[j] = a.alpha[j];
+        beta[j] = first[j] ? T(0) : sums[0][j] / a.rho_prev[j];
+        upd[j] = open && !first[j];
+        dir[j] = open && !stop;
+        if (blockIdx.x == 0 && threadIdx.x == 0 && upd[j]) {
+            a.rho[j] = sums[0][j];
+            a.err[j] = sums[1][j];
+            if (stop) a.stop[j] = 1;
+            else a.beta[j] = beta[j];
+        }
+    }
     const uint32_t L = xcd_logical_block(blockIdx.x, gridDim.x);
-    const uint32_t k = a.k, G = a.G;
-    const uint32_t g = threadIdx.x / G, j = threadIdx.x % G;
-    if (j >= k || a.done[j]) return;
     uint32_t r0, r1;
     block_rows(a.m, a.rows_per_block, L, r0, r1);
-    if (a.iters[j] == 0) {
-        for (uint32_t row = r0 + g; row < r1; row += kBlock / G) {
-            const uint64_t i = uint64_t(row) * k + j;
-            a.d[i] = a.h[i];
+    constexpr int U = 2;
+    for (uint32_t i0 = r0 + threadIdx.x; i0 < r1; i0 += U * kBlock) {
+        T xv[U][K], dv[U][K], rv[U][K], pv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t i = i0 + uint32_t(u * kBlock);
+            if (i < r1) {
+                __builtin_memcpy(xv[u], a.x + uint64_t(i) * K, sizeof(T) * K);
+                __builtin_memcpy(dv[u], a.d + uint64_t(i) * K, sizeof(T) * K);
+                __builtin_memcpy(rv[u], a.r + uint64_t(i) * K, sizeof(T) * K);
+                pv[u] = PREC ? a.dinv[i] : T(1);
+            }
         }
-    } else {
-        const T beta = a.beta[j];
-        for (uint32_t row = r0 + g; row < r1; row += kBlock / G) {
-            const uint64_t i = uint64_t(row) * k + j;
-            a.d[i] = add_rn(mul_rn(beta, a.d[i]), a.h[i]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t i = i0 + uint32_t(u * kBlock);
+            if (i < r1) {
+#pragma unroll
+                for (int j = 0; j < K; ++j) {
+                    const T h = PREC ? mul_rn(pv[u], rv[u][j]) : rv[u][j];
+                    const T x = add_rn(xv[u][j], mul_rn(-alpha[j], dv[u][j]));
+                    const T d = first[j] ? h : add_rn(mul_rn(beta[j], dv[u][j]), h);
+                    xv[u][j] = upd[j] ? x : xv[u][j];
+                    dv[u][j] = dir[j] ? d : dv[u][j];
+                }
+                __builtin_memcpy(a.x + uint64_t(i) * K, xv[u], sizeof(T) * K);
+                __builtin_memcpy(a.d + uint64_t(i) * K, dv[u], sizeof(T) * K);
+            }
+        }
+    }
+}
+
+// The scalars of the direction step, one workgroup per column (larger k).
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_m_beta(MultiArgs<T> a, int max_iter) {
+    __shared__ T lds[kWavesPerBlock];
+    const uint32_t j = blockIdx.x;
+    const int it = a.iters[j];
+    if (a.done[j] || it == 0) return;
+    const T rho = col_sum(a.part_rh, a.P, a.k, j, lds);
+    const T err = col_sum(a.part_rr, a.P, a.k, j, lds);
+    if (threadIdx.x == 0) {
+        a.rho[j] = rho;
+        a.err[j] = err;
+        if (!(err > a.thresh[j]) || it >= max_iter) a.stop[j] = 1;
+        else a.beta[j] = rho / a.rho_prev[j];
+    }
+}
+
+// Rows per lane and trip of the element-wise steps of larger k: their loads
+// before their stores.
+constexpr int kMultiU = 4;
+
+// Direction step of larger k: V adjacent columns per lane, G / V lanes per row.
+template <int V, typename T, bool PREC>
+__global__ __launch_bounds__(kBlock) void k_m_dir(MultiArgs<T> a) {
+    if (!any_open(a)) return;  // every column has stopped
+    const uint32_t L = xcd_logical_block(blockIdx.x, gridDim.x);
+    const uint32_t k = a.k, lanes = a.G / V, per = kBlock / lanes;
+    const uint32_t g = threadIdx.x / lanes, j = (threadIdx.x % lanes) * V;
+    if (j >= k) return;
+    bool upd[V], dir[V], first[V];
+    T alpha[V], beta[V];
+    bool any = false;
+#pragma unroll
+    for (int c = 0; c < V; ++c) {
+        first[c] = a.iters[j + c] == 0;
+        upd[c] = !a.done[j + c] && !first[c];
+        dir[c] = !a.done[j + c] && !a.stop[j + c];
+        any |= upd[c] || dir[c];
+        alpha[c] = a.alpha[j + c];
+        beta[c] = a.beta[j + c];
+    }
+    if (!any) return;
+    uint32_t r0, r1;
+    block_rows(a.m, a.rows_per_block, L, r0, r1);
+    for (uint32_t i0 = r0 + g; i0 < r1; i0 += kMultiU * per) {
+        Lane<V, T> xv[kMultiU], dv[kMultiU], rv[kMultiU];
+        T pv[kMultiU];
+#pragma unroll
+        for (int u = 0; u < kMultiU; ++u) {
+            const uint32_t row = i0 + uint32_t(u) * per;
+            if (row < r1) {
+                const uint64_t i = uint64_t(row) * k + j;
+                xv[u] = lane_load<V>(a.x + i);
+                dv[u] = lane_load<V>(a.d + i);
+                rv[u] = lane_load<V>(a.r + i);
+                pv[u] = PREC ? a.dinv[row] : T(1);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kMultiU; ++u) {
+            const uint32_t row = i0 + uint32_t(u) * per;
+            if (row < r1) {
+                const uint64_t i = uint64_t(row) * k + j;
+#pragma unroll
+                for (int c = 0; c < V; ++c) {
+                    const T h = PREC ? mul_rn(pv[u], rv[u].v[c]) : rv[u].v[c];
+                    const T x = add_rn(xv[u].v[c], mul_rn(-alpha[c], dv[u].v[c]));
+                    const T d = first[c] ? h : add_rn(mul_rn(beta[c], dv[u].v[c]), h);
+                    xv[u].v[c] = upd[c] ? x : xv[u].v[c];
+                    dv[u].v[c] = dir[c] ? d : dv[u].v[c];
+                }
+                __builtin_memcpy(a.x + i, xv[u].v, sizeof(T) * V);
+                __builtin_memcpy(a.d + i, dv[u].v, sizeof(T) * V);
+            }
         }
     }
 }
@@ -195,6 +363,7 @@ __global__ __launch_bounds__(kBlock) void k_m_dir(MultiArgs<T> a) {
 template <int G, int V, typename T>
 __global__ __launch_bounds__(kBlock) void k_m_spmm(MultiArgs<T> a) {
     __shared__ T lds[kBlock * V];
+    close_stopped(a);
     if (!any_active(a)) return;  // every column has stopped (block-uniform)
     const uint32_t L = xcd_logical_block(blockIdx.x, gridDim.x);
     const uint32_t k = a.k;
@@ -246,7 +415,9 @@ struct MultiDqEpilogue {
 // then the wavefronts in index order; out[j] for j < K.  Every thread of
 // the block calls it (it synchronises the block).
 template <int K, typename T>
-__device__ __forceinline__ void stream_partials(const T (&v)[K], T* red, T* out) {
+__device__ __forceinline__ void stream_partials(const T (&v)[K], T* red, T* out,
+                                                const int32_t* done = nullptr,
+                                                const int32_t* stop = nullptr) {
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     __syncthreads();  // red of an earlier call has been read
 #pragma unroll
@@ -255,7 +426,8 @@ __device__ __forceinline__ void stream_partials(const T (&v)[K], T* red, T* out)
         if (lane == 0) red[w * K + j] = s;
     }
     __syncthreads();
-    if (threadIdx.x < uint32_t(K)) {
+    // a stopped column's partials stay as they are (see column_partials_v)
+    if (threadIdx.x < uint32_t(K) && !(done && (done[threadIdx.x] || stop[threadIdx.x]))) {
         T s = red[threadIdx.x];
         for (int x = 1; x < kWavesPerBlock; ++x) s += red[x * K + threadIdx.x];
         out[threadIdx.x] = s;
@@ -269,13 +441,14 @@ __global__ __launch_bounds__(kBlock) void k_m_spmm_stream(MultiArgs<T> a) {
     using Eng = MultiStreamEngine<K, kMultiStreamE, D16>;
     __shared__ T stage[kWavesPerBlock * Eng::kStage];
     __shared__ T red[kWavesPerBlock * K];
+    close_stopped(a);
     if (!any_active(a)) return;  // every column has stopped (block-uniform)
     const uint32_t L = xcd_logical_block(blockIdx.x, gridDim.x);
     bool act[K];
     T pdq[K];
 #pragma unroll
     for (int j = 0; j < K; ++j) {
-        act[j] = !a.done[j];
+        act[j] = !a.done[j] && !a.stop[j];
         pdq[j] = T(0);
     }
     MultiDqEpilogue<K, T> epi{a.d, a.q, pdq};
@@ -283,8 +456,8 @@ __global__ __launch_bounds__(kBlock) void k_m_spmm_stream(MultiArgs<T> a) {
     stream_partials<K>(pdq, red, a.part_dq + size_t(L) * K);
 }
 
-// The start's epilogue (k_m_init's, row by row): r = A x - b, h = D^-1 r,
-// partials of r.h, r.r and b.b per column.
+// The start's epilogue (k_m_init's, row by row): r = A x - b and, with
+// h = D^-1 r, partials of r.h, r.r and b.b per column.
 template <int K, typename T, bool PREC>
 struct MultiInitEpilogue {
     const MultiArgs<T>& a;
@@ -310,7 +483,6 @@ struct MultiInitEpilogue {
             const T ri = add_rn(s[j], mul_rn(T(-1), bi));
             const T hi = PREC ? mul_rn(pv.dinv, ri) : ri;
             a.r[i] = ri;
-            a.h[i] = hi;
             prh[j] += ri * hi;
             prr[j] += ri * ri;
             pbb[j] += bi * bi;
@@ -341,113 +513,191 @@ __global__ __launch_bounds__(kBlock) void k_m_init_stream(MultiArgs<T> a) {
     stream_partials<K>(pbb, red, a.part_bb + size_t(L) * K);
 }
 
+// The scalars of the update step, one workgroup per column (larger k).
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_m_reduce_alpha(MultiArgs<T> a) {
+__global__ __launch_bounds__(kBlock) void k_m_alpha(MultiArgs<T> a) {
     __shared__ T lds[kWavesPerBlock];
     const uint32_t j = blockIdx.x;
-    if (a.done[j]) return;
+    if (a.done[j] || a.stop[j]) return;
     const T dq = col_sum(a.part_dq, a.Pdq, a.k, j, lds);
-    if (threadIdx.x == 0) a.alpha[j] = a.rho[j] / dq;
+    if (threadIdx.x == 0) {
+        const T rho = a.rho[j];
+        a.alpha[j] = rho / dq;
+        a.rho_prev[j] = rho;
+        a.iters[j] = a.iters[j] + 1;
+    }
 }
 
-template <typename T, bool PREC>
-__global__ __launch_bounds__(kBlock) void k_m_update(MultiArgs<T> a) {
-    __shared__ T lds[kBlock];
+// Update step for K <= kMultiStreamMaxK columns, one row per lane: alpha of
+// every column from the SpMM's partials (block 0 writes the scalars), then r.
+template <int K, typename T, bool PREC>
+__global__ __launch_bounds__(kBlock) void k_m_update_few(MultiArgs<T> a) {
+    __shared__ T lds[kWavesPerBlock * K];
+    __shared__ T red[kWavesPerBlock * K];
     if (!any_active(a)) return;  // every column has stopped (block-uniform)
+    T dq[1][K];
+    const T* const parts[1] = {a.part_dq};
+    all_col_sums<1, K>(parts, a.Pdq, lds, dq);
+    bool act[K];
+    T alpha[K], prh[K], prr[K];
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        act[j] = !a.done[j] && !a.stop[j];
+        const T rho = a.rho[j];
+        alpha[j] = rho / dq[0][j];
+        prh[j] = prr[j] = T(0);
+        if (blockIdx.x == 0 && threadIdx.x == 0 && act[j]) {
+            a.alpha[j] = alpha[j];
+            a.rho_prev[j] = rho;
+            a.iters[j] = a.iters[j] + 1;
+        }
+    }
     const uint32_t L = xcd_logical_block(blockIdx.x, gridDim.x);
-    const uint32_t k = a.k;
-    // element-wise over the same rows as the SpMM block, G lanes per row
-    const uint32_t G = a.G;
-    const uint32_t g = threadIdx.x / G, j = threadIdx.x % G;
     uint32_t r0, r1;
     block_rows(a.m, a.rows_per_block, L, r0, r1);
-    T prh = T(0), prr = T(0);
-    if (j < k && !a.done[j]) {
-        const T alpha = a.alpha[j];
-        for (uint32_t row = r0 + g; row < r1; row += kBlock / G) {
-            const uint64_t i = uint64_t(row) * k + j;
-            const T xi = add_rn(a.x[i], mul_rn(-alpha, a.d[i]));
-            const T ri = add_rn(a.r[i], mul_rn(-alpha, a.q[i]));
-            const T hi = PREC ? mul_rn(a.dinv[row], ri) : ri;
-            a.x[i] = xi;
-            a.r[i] = ri;
-            a.h[i] = hi;
-            prh += ri * hi;
-            prr += ri * ri;
+    constexpr int U = 2;
+    for (uint32_t i0 = r0 + threadIdx.x; i0 < r1; i0 += U * kBlock) {
+        T rv[U][K], qv[U][K], pv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t i = i0 + uint32_t(u * kBlock);
+            if (i < r1) {
+                __builtin_memcpy(rv[u], a.r + uint64_t(i) * K, sizeof(T) * K);
+                __builtin_memcpy(qv[u], a.q + uint64_t(i) * K, sizeof(T) * K);
+                pv[u] = PREC ? a.dinv[i] : T(1);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t i = i0 + uint32_t(u * kBlock);
+            if (i < r1) {
+#pragma unroll
+                for (int j = 0; j < K; ++j) {
+                    const T ri = add_rn(rv[u][j], mul_rn(-alpha[j], qv[u][j]));
+                    const T hi = PREC ? mul_rn(pv[u], ri) : ri;
+                    rv[u][j] = act[j] ? ri : rv[u][j];
+                    prh[j] += ri * hi;
+                    prr[j] += ri * ri;
+                }
+                __builtin_memcpy(a.r + uint64_t(i) * K, rv[u], sizeof(T) * K);
+            }
         }
     }
-    column_partials(prh, k, G, lds, a.part_rh + size_t(L) * k);
-    column_partials(prr, k, G, lds, a.part_rr + size_t(L) * k);
+    stream_partials<K>(prh, red, a.part_rh + size_t(L) * K, a.done, a.stop);
+    stream_partials<K>(prr, red, a.part_rr + size_t(L) * K, a.done, a.stop);
 }
 
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_m_reduce_beta(MultiArgs<T> a, int max_iter) {
-    __shared__ T lds[kWavesPerBlock];
-    const uint32_t j = blockIdx.x;
-    if (a.done[j]) return;
-    const T rho_new = col_sum(a.part_rh, a.P, a.k, j, lds);
-    const T err = col_sum(a.part_rr, a.P, a.k, j, lds);
-    if (threadIdx.x == 0) {
-        const int it = a.iters[j] + 1;
-        a.iters[j] = it;
-        a.err[j] = err;
-        if (!(err > a.thresh[j]) || it >= max_iter) {
-            a.done[j] = 1;
-        } else {
-            a.beta[j] = rho_new / a.rho[j];
-            a.rho[j] = rho_new;
+// Update step of larger k: V adjacent columns per lane, G / V lanes per row.
+template <int V, typename T, bool PREC>
+__global__ __launch_bounds__(kBlock) void k_m_update(MultiArgs<T> a) {
+    __shared__ T lds[kBlock * V];
+    if (!any_active(a)) return;  // every column has stopped (block-uniform)
+    const uint32_t L = xcd_logical_block(blockIdx.x, gridDim.x);
+    const uint32_t k = a.k, lanes = a.G / V, per = kBlock / lanes;
+    const uint32_t g = threadIdx.x / lanes, j = (threadIdx.x % lanes) * V;
+    T prh[V], prr[V], alpha[V];
+    bool act[V];
+    bool any = false;
+#pragma unroll
+    for (int c = 0; c < V; ++c) {
+        prh[c] = prr[c] = alpha[c] = T(0);
+        act[c] = j + c < k && !a.done[j + c] && !a.stop[j + c];
+        if (act[c]) alpha[c] = a.alpha[j + c];
+        any |= act[c];
+    }
+    uint32_t r0, r1;
+    block_rows(a.m, a.rows_per_block, L, r0, r1);
+    if (any) {
+        for (uint32_t i0 = r0 + g; i0 < r1; i0 += kMultiU * per) {
+            Lane<V, T> rv[kMultiU], qv[kMultiU];
+            T pv[kMultiU];
+#pragma unroll
+            for (int u = 0; u < kMultiU; ++u) {
+                const uint32_t row = i0 + uint32_t(u) * per;
+                if (row < r1) {
+                    const uint64_t i = uint64_t(row) * k + j;
+                    rv[u] = lane_load<V>(a.r + i);
+                    qv[u] = lane_load<V>(a.q + i);
+                    pv[u] = PREC ? a.dinv[row] : T(1);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kMultiU; ++u) {
+                const uint32_t row = i0 + uint32_t(u) * per;
+                if (row < r1) {
+                    const uint64_t i = uint64_t(row) * k + j;
+#pragma unroll
+                    for (int c = 0; c < V; ++c) {
+                        const T ri = add_rn(rv[u].v[c], mul_rn(-alpha[c], qv[u].v[c]));
+                        const T hi = PREC ? mul_rn(pv[u], ri) : ri;
+                        rv[u].v[c] = act[c] ? ri : rv[u].v[c];
+                        prh[c] += ri * hi;
+                        prr[c] += ri * ri;
+                    }
+                    __builtin_memcpy(a.r + i, rv[u].v, sizeof(T) * V);
+                }
+            }
         }
     }
+    column_partials_v<V>(prh, k, lanes, lds, a.part_rh + size_t(L) * k, a.done, a.stop);
+    column_partials_v<V>(prr, k, lanes, lds, a.part_rr + size_t(L) * k, a.done, a.stop);
 }
 
-// Re-opens the columns flagged in `again` (their loop stopped on the
-// stopping test; the host has lowered their thresholds): the reduction the
-// stopping launch skipped (rho_new from the r.h partials, beta = rho_new /
-// rho, rho = rho_new) and done = 0.  The next launches continue those
-// columns exactly as if their threshold had been the lower one from the
-// start.
+// Re-opens the columns flagged in `again` (their loop stopped on the stopping
+// test; the host has lowered their thresholds).  alpha = 0: the direction
+// step that stopped has applied the pending x -= alpha d.  The next one
+// recomputes rho and err from the same partials and, the test failing now,
+// goes on as it would have with this threshold from the start.
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_m_reopen(MultiArgs<T> a, const int32_t* again) {
-    __shared__ T lds[kWavesPerBlock];
-    const uint32_t j = blockIdx.x;
-    if (!again[j]) return;  // block-uniform
-    const T rho_new = col_sum(a.part_rh, a.P, a.k, j, lds);
-    if (threadIdx.x == 0) {
-        a.beta[j] = rho_new / a.rho[j];
-        a.rho[j] = rho_new;
-        a.done[j] = 0;
-    }
+__global__ void k_m_reopen(MultiArgs<T> a, const int32_t* again) {
+    const uint32_t j = threadIdx.x;
+    if (j >= a.k || !again[j]) return;
+    a.alpha[j] = T(0);
+    a.stop[j] = 0;
+    a.done[j] = 0;
 }
-
 
 // ---------------------------------------------------- layout / refinement
 
-// interleaved[i*k + j] = colmajor[j*n + i] (and back), G-lane groups per
-// row (G = k rounded up to a power of two), grid-stride over rows.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_to_interleaved(uint32_t n, uint32_t k, uint32_t G,
-                                                           const T* __restrict__ cm,
-                                                           T* __restrict__ il,
-                                                           int32_t* nonzero) {
-    const uint32_t g = threadIdx.x / G, j = threadIdx.x % G, per = kBlock / G;
-    if (j >= k) return;
-    bool nz = false;
-    for (uint64_t i = uint64_t(blockIdx.x) * per + g; i < n; i += uint64_t(gridDim.x) * per) {
-        const T v = cm[uint64_t(j) * n + i];
-        il[i * k + j] = v;
-        nz |= !(v == T(0));
-    }
-    if (nonzero && nz) *nonzero = 1;  // every writer stores 1
-}
+// interleaved[i*k + j] = colmajor[j*n + i] and back, in tiles of kLayoutRows
+// rows through LDS (rows padded to an odd length): runs of 512 bytes per
+// column on one side, whole rows on the other.  For 2.25 M rows and 32 columns
+// 228 us in and 202 us out (368 and 557 us with a group of lanes per row).
+constexpr uint32_t kLayoutRows = 64;
 
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_to_colmajor(uint32_t n, uint32_t k, uint32_t G,
-                                                        const T* __restrict__ il,
-                                                        T* __restrict__ cm) {
-    const uint32_t g = threadIdx.x / G, j = threadIdx.x % G, per = kBlock / G;
-    if (j >= k) return;
-    for (uint64_t i = uint64_t(blockIdx.x) * per + g; i < n; i += uint64_t(gridDim.x) * per)
-        cm[uint64_t(j) * n + i] = il[i * k + j];
+template <typename T, bool IN>
+__global__ __launch_bounds__(kBlock) void k_layout(uint32_t n, uint32_t k,
+                                                   const T* __restrict__ src,
+                                                   T* __restrict__ dst, int32_t* nonzero) {
+    __shared__ T tile[kLayoutRows * 33];
+    const uint32_t ld = k | 1u;
+    bool nz = false;
+    const uint64_t step = uint64_t(gridDim.x) * kLayoutRows;
+    for (uint64_t r0 = uint64_t(blockIdx.x) * kLayoutRows; r0 < n; r0 += step) {
+        const uint32_t rows = n - r0 < kLayoutRows ? uint32_t(n - r0) : kLayoutRows;
+        const uint32_t row = threadIdx.x % kLayoutRows;
+        __syncthreads();  // the previous tile has been written
+        if (IN) {
+            for (uint32_t j = threadIdx.x / kLayoutRows; j < k; j += kBlock / kLayoutRows)
+                if (row < rows) {
+                    const T v = src[uint64_t(j) * n + r0 + row];
+                    tile[row * ld + j] = v;
+                    nz |= !(v == T(0));
+                }
+        } else {
+            for (uint32_t e = threadIdx.x; e < rows * k; e += kBlock)
+                tile[(e / k) * ld + e % k] = src[r0 * k + e];
+        }
+        __syncthreads();
+        if (IN) {
+            for (uint32_t e = threadIdx.x; e < rows * k; e += kBlock)
+                dst[r0 * k + e] = tile[(e / k) * ld + e % k];
+        } else {
+            for (uint32_t j = threadIdx.x / kLayoutRows; j < k; j += kBlock / kLayoutRows)
+                if (row < rows) dst[uint64_t(j) * n + r0 + row] = tile[row * ld + j];
+        }
+    }
+    if (IN && nonzero && nz) *nonzero = 1;  // every writer stores 1
 }
 
 // R = B - A X (FP64, interleaved), per-column partial |r|^2 and |b|^2.
@@ -594,11 +844,6 @@ __global__ __launch_bounds__(kBlock) void k_m_ir_update(MultiArgs<double> a64,
     }
 static_assert(kMultiStreamMaxK == 4, "one case per k up to kMultiStreamMaxK");
 
-static uint32_t ew_grid_m(uint64_t n) {
-    uint64_t g = (n + kBlock - 1) / kBlock;
-    return uint32_t(g > 4096 ? 4096 : (g == 0 ? 1 : g));
-}
-
 namespace {
 template <typename T>
 hipError_t stream_spmm_kernel(uint32_t k, bool d16, const void*& f) {
@@ -661,39 +906,56 @@ hipError_t multi_start(const MultiArgs<T>& a, bool precond, T eps, int max_iter,
     return hipGetLastError();
 }
 
-template <typename T>
-hipError_t multi_iteration(const MultiArgs<T>& a, bool precond, int max_iter, hipStream_t s) {
-    const uint32_t cg = a.k;  // one workgroup per column for the reductions
-    const bool v2 = multi_two_cols<T>(a.k);
-    k_m_dir<T><<<a.P, kBlock, 0, s>>>(a);
+template <typename T, bool PREC>
+static hipError_t multi_iteration_p(const MultiArgs<T>& a, int max_iter, hipStream_t s) {
     if (a.sp) {
+        switch (a.k) {
+            case 1: k_m_dir_few<1, T, PREC><<<a.P, kBlock, 0, s>>>(a, max_iter); break;
+            case 2: k_m_dir_few<2, T, PREC><<<a.P, kBlock, 0, s>>>(a, max_iter); break;
+            case 3: k_m_dir_few<3, T, PREC><<<a.P, kBlock, 0, s>>>(a, max_iter); break;
+            default: k_m_dir_few<4, T, PREC><<<a.P, kBlock, 0, s>>>(a, max_iter); break;
+        }
         NLHIP_KD_SWITCH(a.k, a.cols.ci16 != nullptr,
                         (k_m_spmm_stream<K, D16, T><<<a.Pdq, kBlock, 0, s>>>(a)));
-    } else {
-        NLHIP_G_SWITCH(a.G, (v2 ? k_m_spmm<G, two_cols_v<G>(), T><<<a.P, kBlock, 0, s>>>(a)
-                               : k_m_spmm<G, 1, T><<<a.P, kBlock, 0, s>>>(a)));
+        switch (a.k) {
+            case 1: k_m_update_few<1, T, PREC><<<a.P, kBlock, 0, s>>>(a); break;
+            case 2: k_m_update_few<2, T, PREC><<<a.P, kBlock, 0, s>>>(a); break;
+            case 3: k_m_update_few<3, T, PREC><<<a.P, kBlock, 0, s>>>(a); break;
+            default: k_m_update_few<4, T, PREC><<<a.P, kBlock, 0, s>>>(a); break;
+        }
+        return hipGetLastError();
     }
-    k_m_reduce_alpha<T><<<cg, kBlock, 0, s>>>(a);
-    if (precond) k_m_update<T, true><<<a.P, kBlock, 0, s>>>(a);
-    else k_m_update<T, false><<<a.P, kBlock, 0, s>>>(a);
-    k_m_reduce_beta<T><<<cg, kBlock, 0, s>>>(a, max_iter);
+    const bool v2 = multi_two_cols<T>(a.k);
+    k_m_beta<T><<<a.k, kBlock, 0, s>>>(a, max_iter);
+    if (v2) k_m_dir<2, T, PREC><<<a.P, kBlock, 0, s>>>(a);
+    else k_m_dir<1, T, PREC><<<a.P, kBlock, 0, s>>>(a);
+    NLHIP_G_SWITCH(a.G, (v2 ? k_m_spmm<G, two_cols_v<G>(), T><<<a.P, kBlock, 0, s>>>(a)
+                           : k_m_spmm<G, 1, T><<<a.P, kBlock, 0, s>>>(a)));
+    k_m_alpha<T><<<a.k, kBlock, 0, s>>>(a);
+    if (v2) k_m_update<2, T, PREC><<<a.P, kBlock, 0, s>>>(a);
+    else k_m_update<1, T, PREC><<<a.P, kBlock, 0, s>>>(a);
     return hipGetLastError();
+}
+
+template <typename T>
+hipError_t multi_iteration(const MultiArgs<T>& a, bool precond, int max_iter, hipStream_t s) {
+    return precond ? multi_iteration_p<T, true>(a, max_iter, s)
+                   : multi_iteration_p<T, false>(a, max_iter, s);
 }
 
 template <typename T>
 hipError_t multi_layout(uint32_t n, uint32_t k, const T* src, T* dst, bool to_interleaved,
                         hipStream_t s, int32_t* nonzero) {
     if (k == 0 || k > 32) return hipErrorInvalidValue;
-    uint32_t G = 1;
-    while (G < k) G <<= 1;
-    const uint32_t g = ew_grid_m(uint64_t(n) * G);
-    if (to_interleaved) k_to_interleaved<T><<<g, kBlock, 0, s>>>(n, k, G, src, dst, nonzero);
-    else k_to_colmajor<T><<<g, kBlock, 0, s>>>(n, k, G, src, dst);
+    const uint64_t tiles = (uint64_t(n) + kLayoutRows - 1) / kLayoutRows;
+    const uint32_t g = uint32_t(tiles < 16384 ? (tiles ? tiles : 1) : 16384);
+    if (to_interleaved) k_layout<T, true><<<g, kBlock, 0, s>>>(n, k, src, dst, nonzero);
+    else k_layout<T, false><<<g, kBlock, 0, s>>>(n, k, src, dst, nullptr);
     return hipGetLastError();
 }
 
 hipError_t multi_reopen(const MultiArgs<double>& a, const int32_t* again, hipStream_t s) {
-    k_m_reopen<double><<<a.k, kBlock, 0, s>>>(a, again);
+    k_m_reopen<double><<<1, kWave, 0, s>>>(a, again);
     return hipGetLastError();
 }
 
@@ -723,13 +985,20 @@ hipError_t multi_ir_update(const MultiArgs<double>& a64, const MultiArgs<float>&
 }
 
 // dst[:, j] = src[:, j] for the columns j with flag[j] (interleaved n x k).
-__global__ __launch_bounds__(kBlock) void k_m_copy_cols(uint64_t nk, uint32_t k,
+__global__ __launch_bounds__(kBlock) void k_m_copy_cols(uint32_t n, uint32_t k,
                                                         double* __restrict__ dst,
                                                         const double* __restrict__ src,
                                                         const int32_t* __restrict__ flag) {
+    const uint64_t nk = uint64_t(n) * k;
     const uint64_t stride = uint64_t(gridDim.x) * kBlock;
-    for (uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x; i < nk; i += stride)
-        if (flag[i % k]) dst[i] = src[i];
+    uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
+    uint32_t j = uint32_t(i % k);
+    const uint32_t dj = uint32_t(stride % k);
+    for (; i < nk; i += stride) {
+        if (flag[j]) dst[i] = src[i];
+        j += dj;
+        j -= j >= k ? k : 0u;
+    }
 }
 
 hipError_t multi_copy_cols(uint32_t n, uint32_t k, double* dst, const double* src,
@@ -737,7 +1006,7 @@ hipError_t multi_copy_cols(uint32_t n, uint32_t k, double* dst, const double* sr
     const uint64_t nk = uint64_t(n) * k;
     if (nk == 0) return hipSuccess;
     const uint64_t g = (nk + kBlock - 1) / kBlock;
-    k_m_copy_cols<<<uint32_t(g < 16384 ? g : 16384), kBlock, 0, s>>>(nk, k, dst, src, flag);
+    k_m_copy_cols<<<uint32_t(g < 16384 ? g : 16384), kBlock, 0, s>>>(n, k, dst, src, flag);
     return hipGetLastError();
 }
 

@@ -179,6 +179,10 @@ class PinnedBuf {
 // True when p is device (or managed) memory the GPU can address directly.
 bool is_device_pointer(const void* p);
 
+// True when p is plain memory of the device in use, which its kernels may read
+// in place.
+bool on_this_device(const void* p);
+
 // Copies n elements into a device buffer from a host or device pointer.
 void copy_in(void* dst, const void* src, size_t bytes, hipStream_t s);
 // Copies n elements from device to a host or device pointer.
@@ -372,8 +376,8 @@ struct CGWorkspace {
 template <typename T>
 struct MultiWork {
     uint32_t n = 0, k = 0, P = 0;
-    DevBuf<T> x, b, r, h, d, q, part, col;  // part: 4 x P x k; col: 6 x k
-    DevBuf<int32_t> iters, done, skip, again;
+    DevBuf<T> x, b, r, d, q, part, col;     // part: 4 x max(P, Pdq) x k; col: 7 x k
+    DevBuf<int32_t> iters, done, stop, skip, again;
     DevBuf<int32_t> xnz;                    // X has a nonzero (args.x_nonzero)
     DevBuf<T> chk;                          // 2 x k: |b - A x|^2, |b|^2 (confirm)
     PinnedBuf<int32_t> host;                // two polling slots of 32 done flags

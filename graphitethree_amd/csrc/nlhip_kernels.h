@@ -316,14 +316,14 @@ struct MultiArgs {
     T* x;                     // n x k interleaved
     const T* b;
     T* r;
-    T* h;
     T* d;
     T* q;
-    T* part_dq;               // P x k
-    T* part_rh;
+    T* part_dq;               // Pdq x k
+    T* part_rh;               // P x k (the start's: Pdq x k)
     T* part_rr;
     T* part_bb;
     T* rho;                   // per column
+    T* rho_prev;
     T* alpha;
     T* beta;
     T* err;
@@ -331,6 +331,7 @@ struct MultiArgs {
     T* bb;
     int32_t* iters;
     int32_t* done;
+    int32_t* stop;            // the test held (done from the next SpMM on)
     const int32_t* skip;      // may be null
     // null, or a flag that reads 0 when X is all zeros: the start then takes
     // every row sum of A X as +0 without reading the matrix (the sum of
@@ -364,8 +365,7 @@ hipError_t multi_iteration(const MultiArgs<T>& a, bool precond, int max_iter, hi
 template <typename T>
 hipError_t multi_layout(uint32_t n, uint32_t k, const T* src, T* dst, bool to_interleaved,
                         hipStream_t s, int32_t* nonzero = nullptr);
-// Re-opens the FP64 columns flagged in again[k] (done -> 0 with the beta /
-// rho update their stopping launch skipped), then recounts the active ones.
+// Re-opens the FP64 columns flagged in again[k] (their thresholds lowered).
 hipError_t multi_reopen(const MultiArgs<double>& a, const int32_t* again, hipStream_t s);
 hipError_t multi_residual64(const MultiArgs<double>& a, hipStream_t s);
 hipError_t multi_scale_cast(const MultiArgs<double>& a64, const MultiArgs<float>& a32,

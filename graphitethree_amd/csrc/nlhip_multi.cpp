@@ -21,17 +21,20 @@ uint32_t pow2_ceil(uint32_t k) {
     return g;
 }
 
-// Workgroups of the multi right-hand-side launches: enough for one pass of
-// G-lane row groups over the matrix; at most 16 per CU when the SpMM step
-// streams (it has its own count), otherwise as many as the row engine's SpMM
-// step keeps resident (its workgroups take neighbouring rows in turn, so the
-// ones that wait for a place would come back to rows that have left the L2).
+// Workgroups of the multi right-hand-side launches.  k <= kMultiStreamMaxK
+// (the element-wise steps; the streamed SpMM has its own count): a row per
+// lane, at most 4 per CU, because every one of them adds up the partials of
+// all.  Larger k: enough for one pass of the row groups, at most as many as the
+// row engine's SpMM step keeps resident (its workgroups take neighbouring rows
+// in turn, so the ones that wait for a place would come back to rows that have
+// left the L2).
 template <typename T>
 uint32_t multi_grid(const System& S, uint32_t k) {
-    const uint32_t per = 256u / pow2_ceil(k);
+    const bool few = k <= kMultiStreamMaxK;
+    const uint32_t per = few ? 256u : 256u / pow2_ceil(k);
     const uint64_t passes = (uint64_t(S.n) + per - 1) / per;
-    const uint64_t cap = uint64_t(std::max(1, device().cu_count)) *
-                         (k <= kMultiStreamMaxK ? 16u : multi_rows_per_cu<T>(k));
+    const uint64_t cap =
+        uint64_t(std::max(1, device().cu_count)) * (few ? 4u : multi_rows_per_cu<T>(k));
     return uint32_t(std::max<uint64_t>(1, std::min(passes, cap)));
 }
 
@@ -47,11 +50,10 @@ void multi_alloc(System& S, MultiWork<T>& w, uint32_t k) {
     w.x.alloc(nk);
     w.b.alloc(nk);
     w.r.alloc(nk);
-    w.h.alloc(nk);
     w.d.alloc(nk);
     w.q.alloc(nk);
-    w.part.alloc(4 * size_t(P) * k);
-    w.col.alloc(6 * size_t(k));
+    w.col.alloc(7 * size_t(k));
+    w.stop.alloc(k);
     w.iters.alloc(k);
     w.done.alloc(k);
     w.skip.alloc(k);
@@ -69,10 +71,7 @@ void multi_alloc(System& S, MultiWork<T>& w, uint32_t k) {
     a.k = k;
     a.G = pow2_ceil(k);
     a.P = P;
-    const uint32_t rows_per_pass = 256u / a.G;
-    uint64_t rpb = (uint64_t(S.n) + P - 1) / P;
-    rpb = (rpb + rows_per_pass - 1) / rows_per_pass * rows_per_pass;
-    a.rows_per_block = uint32_t(std::max<uint64_t>(rpb, rows_per_pass));
+    a.rows_per_block = uint32_t((uint64_t(S.n) + P - 1) / P);
     a.rp = S.rowptr.get();
     a.ci = S.colind.get();
     a.cols = S.cols();
@@ -80,11 +79,11 @@ void multi_alloc(System& S, MultiWork<T>& w, uint32_t k) {
     if (k <= kMultiStreamMaxK) {
         // stream SpMM: the 64-row tiles dealt to as many workgroups as the
         // device holds at once (no second, partly filled round), a multiple
-        // of 4 tiles (one quarter per wavefront) to each, at most P workgroups
+        // of 4 tiles (one quarter per wavefront) to each
         const uint64_t ntiles = (uint64_t(S.n) + 63) / 64;
         const uint64_t resident = uint64_t(std::max(1, device().cu_count)) *
                                   multi_stream_per_cu<T>(k, a.cols.ci16 != nullptr);
-        const uint64_t want = std::min<uint64_t>({P, resident, (ntiles + 3) / 4});
+        const uint64_t want = std::min<uint64_t>(resident, (ntiles + 3) / 4);
         uint64_t sp = (ntiles + want - 1) / want;
         sp = (sp + 3) / 4 * 4;
         a.sp = uint32_t(sp);
@@ -93,19 +92,22 @@ void multi_alloc(System& S, MultiWork<T>& w, uint32_t k) {
     a.x = w.x.get();
     a.b = w.b.get();
     a.r = w.r.get();
-    a.h = w.h.get();
     a.d = w.d.get();
     a.q = w.q.get();
+    const size_t parts = size_t(std::max(P, a.Pdq)) * k;
+    w.part.alloc(4 * parts);
     a.part_dq = w.part.get();
-    a.part_rh = w.part.get() + size_t(P) * k;
-    a.part_rr = w.part.get() + 2 * size_t(P) * k;
-    a.part_bb = w.part.get() + 3 * size_t(P) * k;
+    a.part_rh = w.part.get() + parts;
+    a.part_rr = w.part.get() + 2 * parts;
+    a.part_bb = w.part.get() + 3 * parts;
     a.rho = w.col.get();
     a.alpha = w.col.get() + k;
     a.beta = w.col.get() + 2 * size_t(k);
     a.err = w.col.get() + 3 * size_t(k);
     a.thresh = w.col.get() + 4 * size_t(k);
     a.bb = w.col.get() + 5 * size_t(k);
+    a.rho_prev = w.col.get() + 6 * size_t(k);
+    a.stop = w.stop.get();
     a.iters = w.iters.get();
     a.done = w.done.get();
     a.skip = nullptr;
@@ -226,12 +228,16 @@ void solve_multi(System& S, uint32_t k, const double* B, double* X, const nlhip_
     multi_alloc(S, S.m64, k);
     MultiWork<double>& w = S.m64;
     const size_t nk = size_t(S.n) * k;
-    // stage column-major B and X through q, then interleave
-    copy_in(w.q.get(), B, nk * 8, s);
-    NLHIP_CHECK(multi_layout<double>(S.n, k, w.q.get(), w.b.get(), true, s));
-    copy_in(w.q.get(), X, nk * 8, s);
-    NLHIP_CHECK(hipMemsetAsync(w.xnz.get(), 0, sizeof(int32_t), s));
-    NLHIP_CHECK(multi_layout<double>(S.n, k, w.q.get(), w.x.get(), true, s, w.xnz.get()));
+    // interleave column-major B and X, from where they are when that is this
+    // device's memory, else staged through q
+    auto staged = [&](const double* p) {
+        if (on_this_device(p)) return p;
+        copy_in(w.q.get(), p, nk * 8, s);
+        return const_cast<const double*>(w.q.get());
+    };
+    NLHIP_CHECK(multi_layout<double>(S.n, k, staged(B), w.b.get(), true, s));
+    NLHIP_CHECK(fill<int32_t>(1, 0, w.xnz.get(), s));
+    NLHIP_CHECK(multi_layout<double>(S.n, k, staged(X), w.x.get(), true, s, w.xnz.get()));
     const bool precond = p.precond == NL_PRECOND_JACOBI;
     const uint32_t K = p.check_every ? p.check_every : multi_check_every(S, k);
     Event e0, e1;
@@ -241,6 +247,8 @@ void solve_multi(System& S, uint32_t k, const double* B, double* X, const nlhip_
     std::vector<double> cgrel(k, 0.0);
     std::vector<uint8_t> conv(k, 0);
     std::vector<uint32_t> first(k, ~0u), extra(k, 0);
+    // |b - A x|^2 and |b|^2 of the result, where the solve ends with them
+    std::vector<double> rr_end, bb_end;
     if (p.precision == NLHIP_PREC_FP64) {
         w.args.val = S.val.get();
         w.args.dinv = precond ? S.dinv.get() : nullptr;
@@ -299,6 +307,8 @@ void solve_multi(System& S, uint32_t k, const double* B, double* X, const nlhip_
                                 : (!(err[j] > thr[j]) ? 1 : 0);
             extra[j] = first[j] == ~0u ? 0u : uint32_t(its[j]) - first[j];
         }
+        rr_end = rr;
+        bb_end = tb;
     } else if (p.precision == NLHIP_PREC_MIXED) {
         S.ensure_fp32();
         multi_alloc(S, S.m32, k);
@@ -379,7 +389,11 @@ void solve_multi(System& S, uint32_t k, const double* B, double* X, const nlhip_
                                            hipMemcpyHostToDevice, s));
                 NLHIP_CHECK(multi_copy_cols(S.n, k, w.x.get(), x_best, w.again.get(), s));
             }
-            if (active == 0) break;
+            if (active == 0) {
+                rr_end = rr;  // of the iterates kept: back at the best where one went on
+                bb_end = bb;
+                break;
+            }
             NLHIP_CHECK(hipMemcpyAsync(w32.skip.get(), skip.data(), k * 4, hipMemcpyHostToDevice, s));
             NLHIP_CHECK(hipMemcpyAsync(S.mscale.get(), sc.data(), sc.size() * 8,
                                        hipMemcpyHostToDevice, s));
@@ -395,10 +409,14 @@ void solve_multi(System& S, uint32_t k, const double* B, double* X, const nlhip_
     e1.record(s);
     e1.sync();
     const double dev_s = 1e-3 * elapsed_ms(e0, e1);
-    std::vector<double> rr, bb;
-    multi_norms(S, k, rr, bb);
-    NLHIP_CHECK(multi_layout<double>(S.n, k, w.x.get(), w.q.get(), false, s));
-    copy_out(X, w.q.get(), nk * 8, s);
+    const std::vector<double>&rr = rr_end, &bb = bb_end;
+    if (rr_end.empty()) multi_norms(S, k, rr_end, bb_end);
+    if (on_this_device(X)) {
+        NLHIP_CHECK(multi_layout<double>(S.n, k, w.x.get(), X, false, s));
+    } else {
+        NLHIP_CHECK(multi_layout<double>(S.n, k, w.x.get(), w.q.get(), false, s));
+        copy_out(X, w.q.get(), nk * 8, s);
+    }
     S.stream.sync();
     const double wall_s =
         std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
