@@ -624,6 +624,8 @@ struct SsorSweepArgs {
     const uint32_t* off;   // first position of each level (levels + 1)
     const uint32_t* eoff;  // first packed entry of each position (n + 1)
     const uint32_t* col;
+    const uint32_t* dep;   // position of each packed entry's row in this sweep
+    const uint32_t* lev;   // level of each position
     const double* val;
 };
 struct SsorArgs {
@@ -638,10 +640,12 @@ struct SsorArgs {
 };
 hipError_t ssor_diag(uint32_t n, const uint32_t* rp, const uint32_t* ci, const double* val,
                      double omega, double* diag, double* dscale, uint32_t* bad, hipStream_t s);
-// Levels [l0, l1) of one sweep; `rows` rows in all (one level: the grid
-// covers them; several levels: one workgroup).
-hipError_t ssor_sweep(const SsorArgs& a, bool upper, uint32_t l0, uint32_t l1, uint32_t rows,
-                      hipStream_t s);
+// One level of a sweep over the whole grid (`rows` rows).
+hipError_t ssor_level(const SsorArgs& a, bool upper, uint32_t l, uint32_t rows, hipStream_t s);
+// The positions [k0, k1) of a sweep, whole levels, by one workgroup
+// (ssor_chain_init first: its LDS size).
+hipError_t ssor_chain_init();
+hipError_t ssor_chain(const SsorArgs& a, bool upper, uint32_t k0, uint32_t k1, hipStream_t s);
 hipError_t ssor_scale(const SsorArgs& a, hipStream_t s);
 
 // An SSOR(omega) preconditioner of a resident matrix (its own copy of the

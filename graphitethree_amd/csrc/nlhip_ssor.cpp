@@ -12,8 +12,9 @@ namespace nlhip {
 
 namespace {
 
-// Levels of at most this many rows run back to back in one workgroup.
-constexpr uint32_t kChainRows = 256;  // one row per thread of a 256-thread workgroup
+// Levels of at most this many rows run back to back in one workgroup: 1024 rows
+// take some 0.7 us, and a launch of its own about 3.
+constexpr uint32_t kChainRows = 4096;
 
 // level(i) = 1 + the deepest level among the rows i reads (j < i for the
 // forward sweep, j > i for the backward one); rows counting-sorted by level
@@ -44,17 +45,18 @@ void level_schedule(uint32_t n, const std::vector<uint32_t>& rp, const std::vect
 
 // One sweep on the device: rows by level and their packed entries.
 struct SweepBufs {
-    DevBuf<uint32_t> rows, off, eoff, col;
+    DevBuf<uint32_t> rows, off, eoff, col, dep, lev;
     DevBuf<double> val;
     SsorSweepArgs args() const {
-        return SsorSweepArgs{rows.get(), off.get(), eoff.get(), col.get(), val.get()};
+        return SsorSweepArgs{rows.get(), off.get(), eoff.get(), col.get(),
+                             dep.get(),  lev.get(), val.get()};
     }
 };
 
 class Ssor {
   public:
     struct Step {
-        uint32_t l0, l1, rows;
+        uint32_t l0, l1, k0, k1;  // levels [l0, l1), positions [k0, k1)
     };
     uint32_t n = 0;
     double omega = 1.5;
@@ -83,8 +85,11 @@ class Ssor {
 
 namespace {
 
-// One launch per level with more than kChainRows rows, one per run of
-// consecutive smaller levels.
+// A level of more than kChainRows rows: over the whole grid.
+bool wide(const Ssor::Step& st) { return st.l1 - st.l0 == 1 && st.k1 - st.k0 > kChainRows; }
+
+// One launch per level with more than kChainRows rows, one workgroup per run
+// of consecutive smaller levels.
 std::vector<Ssor::Step> plan(const std::vector<uint32_t>& off) {
     std::vector<Ssor::Step> steps;
     const uint32_t nl = uint32_t(off.size() - 1);
@@ -92,13 +97,13 @@ std::vector<Ssor::Step> plan(const std::vector<uint32_t>& off) {
     while (l < nl) {
         const uint32_t sz = off[l + 1] - off[l];
         if (sz > kChainRows) {
-            steps.push_back({l, l + 1, sz});
+            steps.push_back({l, l + 1, off[l], off[l + 1]});
             ++l;
             continue;
         }
         uint32_t e = l;
         while (e < nl && off[e + 1] - off[e] <= kChainRows) ++e;
-        steps.push_back({l, e, off[e] - off[l]});
+        steps.push_back({l, e, off[l], off[e]});
         l = e;
     }
     return steps;
@@ -115,31 +120,44 @@ std::vector<Ssor::Step> build_sweep(uint32_t n, const std::vector<uint32_t>& rp,
                                     bool upper, SweepBufs& B, hipStream_t s) {
     std::vector<uint32_t> rows, off;
     level_schedule(n, rp, ci, upper, rows, off);
-    std::vector<uint32_t> eoff(size_t(n) + 1, 0), col;
+    std::vector<Ssor::Step> steps = plan(off);
+    // columns for the levels launched over the grid, positions for the others
+    bool by_col = false, by_pos = false;
+    for (const Ssor::Step& st : steps) (wide(st) ? by_col : by_pos) = true;
+    std::vector<uint32_t> eoff(size_t(n) + 1, 0), col, dep, lev(by_pos ? n : 0), at(by_pos ? n : 0);
     std::vector<double> val;
-    col.reserve(ci.size() / 2 + 1);
     val.reserve(ci.size() / 2 + 1);
+    if (by_col) col.reserve(ci.size() / 2 + 1);
+    if (by_pos) {
+        dep.reserve(ci.size() / 2 + 1);
+        for (uint32_t k = 0; k < n; ++k) at[rows[k]] = k;
+        for (size_t l = 0; l + 1 < off.size(); ++l)
+            std::fill(lev.begin() + off[l], lev.begin() + off[l + 1], uint32_t(l));
+    }
     for (uint32_t k = 0; k < n; ++k) {
         const uint32_t i = rows[k];
         for (uint32_t e = rp[i]; e < rp[i + 1]; ++e)
             if (upper ? ci[e] > i : ci[e] < i) {
-                col.push_back(ci[e]);
+                if (by_col) col.push_back(ci[e]);
+                if (by_pos) dep.push_back(at[ci[e]]);
                 val.push_back(va[e]);
             }
-        eoff[k + 1] = uint32_t(col.size());
+        eoff[k + 1] = uint32_t(val.size());
     }
-    B.rows.alloc(std::max<size_t>(rows.size(), 1));
-    B.off.alloc(off.size());
-    B.eoff.alloc(eoff.size());
-    B.col.alloc(std::max<size_t>(col.size(), 1));
-    B.val.alloc(std::max<size_t>(val.size(), 1));
-    copy_in(B.rows.get(), rows.data(), rows.size() * 4, s);
-    copy_in(B.off.get(), off.data(), off.size() * 4, s);
-    copy_in(B.eoff.get(), eoff.data(), eoff.size() * 4, s);
-    copy_in(B.col.get(), col.data(), col.size() * 4, s);
-    copy_in(B.val.get(), val.data(), val.size() * 8, s);
+    auto put = [&](auto& dst, const auto& src) {
+        if (src.empty()) return;
+        dst.alloc(src.size());
+        copy_in(dst.get(), src.data(), src.size() * sizeof(src[0]), s);
+    };
+    put(B.rows, rows);
+    put(B.off, off);
+    put(B.eoff, eoff);
+    put(B.col, col);
+    put(B.dep, dep);
+    put(B.lev, lev);
+    put(B.val, val);
     NLHIP_CHECK(hipStreamSynchronize(s));  // the host arrays go out of scope
-    return plan(off);
+    return steps;
 }
 
 }  // namespace
@@ -180,11 +198,18 @@ Ssor* ssor_create(System& S, double omega) {
     P->w.alloc(n);
     P->y.alloc(n);
     const SsorArgs a = P->args();
+    NLHIP_CHECK(ssor_chain_init());
     P->graph.capture(s, [&] {
-        for (const Ssor::Step& st : P->lo_steps)
-            NLHIP_CHECK(ssor_sweep(a, false, st.l0, st.l1, st.rows, s));
-        for (const Ssor::Step& st : P->up_steps)
-            NLHIP_CHECK(ssor_sweep(a, true, st.l0, st.l1, st.rows, s));
+        auto sweep = [&](const std::vector<Ssor::Step>& steps, bool upper) {
+            for (const Ssor::Step& st : steps) {
+                if (wide(st))
+                    NLHIP_CHECK(ssor_level(a, upper, st.l0, st.k1 - st.k0, s));
+                else
+                    NLHIP_CHECK(ssor_chain(a, upper, st.k0, st.k1, s));
+            }
+        };
+        sweep(P->lo_steps, false);
+        sweep(P->up_steps, true);
         NLHIP_CHECK(ssor_scale(a, s));
     });
     return P.release();

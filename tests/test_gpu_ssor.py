@@ -209,3 +209,57 @@ def test_context_api_with_ssor(hip):
     assert relr <= 1e-10
     assert rel(gpu[free], xr) <= REL_DIFF
     assert gpu[2 * pins[0]] == uv[0][0]
+
+
+def chain_patterns():
+    rng = np.random.default_rng(12)
+
+    def dominant(A):
+        A = sp.csr_matrix(A)
+        return (A + sp.diags(np.asarray(abs(A).sum(axis=1)).ravel() + 1.0)).tocsr()
+
+    def rows(n, lists):
+        r = np.concatenate([np.full(len(c), i) for i, c in enumerate(lists)])
+        c = np.concatenate(lists).astype(np.int64)
+        return dominant(sp.coo_matrix((rng.standard_normal(len(r)), (r, c)), shape=(n, n)))
+
+    n = 20000
+    arrow = rows(n, [np.array([i % 7, max(i - 1, 0), min(i + 1, n - 1), n - 1 - i % 5])
+                     for i in range(n)])
+    wide = sp.kron(sp.csr_matrix(np.tri(3) + np.tri(3).T), sp.eye(5000)).tocsr()
+    m = 2500
+    long = rows(m, [rng.integers(0, m, 25) for _ in range(m)])
+    # one-row levels, then 6000-row ones, then one-row levels reading both
+    mixed = sp.lil_matrix((9000, 9000))
+    for i in range(1, 9000):
+        if i < 1500 or i >= 7500:
+            mixed[i, i - 1] = 1.0
+        else:
+            mixed[i, 1499 - i % 3] = 0.5
+        if i >= 7500:
+            mixed[i, 1500 + (i * 7) % 6000] = 0.25
+            mixed[i, i % 1000] = -0.5
+    return {"arrow": arrow, "wide_5000": dominant(wide), "long_rows": long,
+            "mixed": dominant(mixed + mixed.T), "one": sp.identity(1, format="csr") * 3.0,
+            "levels_1025": dominant(sp.kron(sp.csr_matrix(np.tri(9) + np.tri(9).T),
+                                            sp.eye(1025)))}
+
+
+@pytest.mark.parametrize("name", ["arrow", "wide_5000", "long_rows", "mixed", "one",
+                                  "levels_1025"])
+def test_chain_edges_are_bitwise_the_oracle(hip, name):
+    """The one-workgroup run of levels: values that have left the LDS ring or
+    come from an earlier launch, levels wider than a chunk, rows of more
+    entries than a lane keeps, runs before and after a level of its own."""
+    A = chain_patterns()[name]
+    M, C = nl_matrix(hip, A)
+    P = hip.nlNewSSORPreconditioner(M, 1.5)
+    assert P
+    x = np.random.default_rng(1).standard_normal(C.m)
+    for _ in range(3):
+        y = np.zeros(C.m)
+        hip.nlMultMatrixVector(P, capi.ptr(x), capi.ptr(y))
+        assert np.array_equal(bits(y), bits(O.ssor(C, x, 1.5)))
+        x = x[::-1].copy()
+    hip.nlDeleteMatrix(P)
+    hip.nlDeleteMatrix(M)
