@@ -161,10 +161,6 @@ __device__ __forceinline__ void block_row_range(uint32_t m, uint32_t chunk, uint
 // the row's tile started, so that the latency of the per-row operands the
 // epilogue reads (b, D^-1, d, ...) overlaps the row's nonzeros.
 
-struct NoPre {
-    __device__ __forceinline__ int operator()(uint32_t) const { return 0; }
-};
-
 template <typename Pre, typename Fin>
 struct Epilogue {
     Pre pre;
@@ -172,17 +168,11 @@ struct Epilogue {
     using PV = decltype(std::declval<Pre&>()(0u));
     template <typename T>
     __device__ __forceinline__ void done(uint32_t row, T sum, const PV& pv) {
-        if constexpr (std::is_same<Pre, NoPre>::value) fin(row, sum);
-        else fin(row, sum, pv);
+        fin(row, sum, pv);
     }
     static constexpr bool kPairs = false;  // see DqEpilogue
 };
 
-// fin(row, sum)
-template <typename Fin>
-__device__ __forceinline__ Epilogue<NoPre, Fin> plain_epi(Fin fin) {
-    return Epilogue<NoPre, Fin>{NoPre{}, fin};
-}
 // pre(row) -> pv; fin(row, sum, pv)
 template <typename Pre, typename Fin>
 __device__ __forceinline__ Epilogue<Pre, Fin> prefetch_epi(Pre pre, Fin fin) {
@@ -219,6 +209,24 @@ struct DqEpilogue {
         *reinterpret_cast<V2*>(q + row) = v;
         pdq += d0 * s0;
         pdq += d1 * s1;
+    }
+};
+
+// y[row] = sum, with the block engine's aligned row pairs as one store each.
+template <typename T>
+struct StoreEpilogue {
+    T* __restrict__ y;
+    using PV = int;
+    using V2 = T __attribute__((ext_vector_type(2)));
+    static constexpr bool kPairs = true;
+    __device__ __forceinline__ int pre(uint32_t) const { return 0; }
+    __device__ __forceinline__ void done(uint32_t row, T sum, int) { y[row] = sum; }
+    __device__ __forceinline__ void pre2(uint32_t, int& a, int& b) const { a = b = 0; }
+    __device__ __forceinline__ void done2(uint32_t row, T s0, T s1, int, int) {
+        V2 v;
+        v.x = s0;
+        v.y = s1;
+        *reinterpret_cast<V2*>(y + row) = v;
     }
 };
 

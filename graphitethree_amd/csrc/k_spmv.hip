@@ -23,7 +23,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv(uint32_t m, uint32_t sp,
                                                  const T* __restrict__ x, T* __restrict__ y) {
     __shared__ T stage[StageSize<RPW>::value];
     const uint32_t L = xcd_logical_block(blockIdx.x, gridDim.x);
-    auto epi = plain_epi([&](uint32_t row, T s) { y[row] = s; });
+    StoreEpilogue<T> epi{y};
     EngineOf<RPW>::type::run(m, sp, L, rp, cols, val, x, stage, epi);
 }
 

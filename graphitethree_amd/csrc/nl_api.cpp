@@ -280,14 +280,7 @@ Precond precond_of(NLMatrix P, uint32_t n) {
 // y = A x for a device system; x, y host or device.
 void system_mult(System* S, const double* x, double* y) {
     std::lock_guard<std::mutex> lock(S->mu);
-    hipStream_t s = S->stream.get();
-    S->ws64.ensure(S->n, S->grid);
-    copy_in(S->ws64.x.get(), x, size_t(S->n) * 8, s);
-    const SpmvOps<double> o = S->ops<double>();
-    NLHIP_CHECK(spmv<double>(S->n, o.rp, o.cols, o.val, S->ws64.x.get(), S->ws64.q.get(), o.code,
-                             S->grid, s));
-    copy_out(y, S->ws64.q.get(), size_t(S->n) * 8, s);
-    S->stream.sync();
+    multiply(*S, x, y);
 }
 
 void dyn_mult(NLMatrix M, const double* x, double* y) {

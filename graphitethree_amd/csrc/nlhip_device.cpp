@@ -100,14 +100,19 @@ bool is_device_pointer(const void* p) {
     return attr.type == hipMemoryTypeDevice || attr.type == hipMemoryTypeManaged;
 }
 
-bool on_this_device(const void* p) {
-    if (!p) return false;
+bool on_this_device(const void* p, size_t bytes, size_t align) {
+    if (!p || reinterpret_cast<uintptr_t>(p) % align) return false;
     hipPointerAttribute_t attr;
-    if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&attr, p) != hipSuccess ||
+        attr.type != hipMemoryTypeDevice || attr.device != device().id ||
+        hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
-    return attr.type == hipMemoryTypeDevice && attr.device == device().id;
+    const size_t at = size_t(static_cast<const char*>(p) - static_cast<const char*>(base));
+    return at <= size && bytes <= size - at;
 }
 
 void copy_in(void* dst, const void* src, size_t bytes, hipStream_t s) {

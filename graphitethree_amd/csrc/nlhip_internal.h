@@ -179,9 +179,10 @@ class PinnedBuf {
 // True when p is device (or managed) memory the GPU can address directly.
 bool is_device_pointer(const void* p);
 
-// True when p is plain memory of the device in use, which its kernels may read
-// in place.
-bool on_this_device(const void* p);
+// True when the bytes at p lie in one plain allocation of the device in use,
+// aligned, so that its kernels may use them in place (a copy would have checked
+// the range).
+bool on_this_device(const void* p, size_t bytes, size_t align);
 
 // Copies n elements into a device buffer from a host or device pointer.
 void copy_in(void* dst, const void* src, size_t bytes, hipStream_t s);
@@ -588,6 +589,9 @@ System* ls_create(uint32_t nvars, uint32_t nrows, const uint32_t* row_ptr, const
                   const uint8_t* locked, const double* values, uint32_t flags, double* rhs,
                   uint32_t* nfree_out);
 void default_launch(uint32_t n, uint64_t nnz, int& rpw, uint32_t& grid);
+
+// y = A x, host or device vectors, complete on return (S.mu held).
+void multiply(System& S, const double* x, double* y);
 
 // |b - A x| / |b| in FP64 on the device.
 double true_rel_residual(System& S, const double* b_dev, const double* x_dev);

@@ -231,7 +231,7 @@ void solve_multi(System& S, uint32_t k, const double* B, double* X, const nlhip_
     // interleave column-major B and X, from where they are when that is this
     // device's memory, else staged through q
     auto staged = [&](const double* p) {
-        if (on_this_device(p)) return p;
+        if (on_this_device(p, nk * 8, 8)) return p;
         copy_in(w.q.get(), p, nk * 8, s);
         return const_cast<const double*>(w.q.get());
     };
@@ -411,7 +411,7 @@ void solve_multi(System& S, uint32_t k, const double* B, double* X, const nlhip_
     const double dev_s = 1e-3 * elapsed_ms(e0, e1);
     const std::vector<double>&rr = rr_end, &bb = bb_end;
     if (rr_end.empty()) multi_norms(S, k, rr_end, bb_end);
-    if (on_this_device(X)) {
+    if (on_this_device(X, nk * 8, 8)) {
         NLHIP_CHECK(multi_layout<double>(S.n, k, w.x.get(), X, false, s));
     } else {
         NLHIP_CHECK(multi_layout<double>(S.n, k, w.x.get(), w.q.get(), false, s));

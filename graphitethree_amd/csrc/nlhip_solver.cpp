@@ -395,6 +395,25 @@ static CGStatus<T> read_status(System& S, CGWorkspace<T>& ws) {
     return st;
 }
 
+// Vectors of this device are used in place: at 10 M rows the two staging
+// copies took 70 of 341 us.  The engines read pairs of x and write pairs of y
+// (16 bytes), and y must not overlap x.
+void multiply(System& S, const double* x, double* y) {
+    hipStream_t s = S.stream.get();
+    const size_t bytes = size_t(S.n) * 8;
+    const bool x_here = on_this_device(x, bytes, 16);
+    const bool apart = x + S.n <= y || y + S.n <= x;
+    const bool y_here = (apart || !x_here) && on_this_device(y, bytes, 16);
+    if (!x_here || !y_here) S.ws64.ensure(S.n, S.grid);
+    if (!x_here) copy_in(S.ws64.x.get(), x, bytes, s);
+    const double* const in = x_here ? x : S.ws64.x.get();
+    double* const out = y_here ? y : S.ws64.q.get();
+    const SpmvOps<double> o = S.ops<double>();
+    NLHIP_CHECK(spmv<double>(S.n, o.rp, o.cols, o.val, in, out, o.code, S.grid, s));
+    if (!y_here) copy_out(y, out, bytes, s);
+    S.stream.sync();
+}
+
 // Reads |b - A x|^2 and |b|^2 (FP64) into rr, bb.
 static void residual_norms(System& S, const double* b, const double* x, double* r_out,
                            double& rr, double& bb) {
@@ -1178,15 +1197,8 @@ NLAPI int NLAPIENTRY nlhipSpMV(nlhip_system s, const double* x, double* y) {
     return guarded("nlhipSpMV", [&] {
         System* S = sys(s);
         std::lock_guard<std::mutex> lock(S->mu);
-        S->pcg.active = false;  // stages through ws64
-        hipStream_t st = S->stream.get();
-        S->ws64.ensure(S->n, S->grid);
-        copy_in(S->ws64.x.get(), x, size_t(S->n) * 8, st);
-        const SpmvOps<double> o = S->ops<double>();
-        NLHIP_CHECK(spmv<double>(S->n, o.rp, o.cols, o.val, S->ws64.x.get(), S->ws64.q.get(),
-                                 o.code, S->grid, st));
-        copy_out(y, S->ws64.q.get(), size_t(S->n) * 8, st);
-        S->stream.sync();
+        S->pcg.active = false;  // may stage through ws64
+        multiply(*S, x, y);
     });
 }
 

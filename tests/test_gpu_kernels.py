@@ -199,6 +199,44 @@ def test_set_launch_rejects_bad_shapes(hip):
             S.set_launch(rpw, wg)
 
 
+@pytest.mark.parametrize("form", ["lscm", "cotan", "odd"])
+def test_spmv_uses_device_vectors_in_place_or_staged(hip, form):
+    """Whole device vectors, ones 8 bytes off the 16-byte grid, the same
+    vector as input and output, overlapping ones and host memory on either
+    side: all are the host result to the bit, and nothing beside y changes."""
+    import torch
+
+    Sw = {"lscm": lambda: W.lscm_grid(31, seed=2),
+          "cotan": lambda: W.cotan_system(W.grid_mesh(40, seed=2), nrhs=1),
+          "odd": lambda: W.cotan_system(W.grid_mesh(33, seed=4), nrhs=1)}[form]()
+    n = Sw.n
+    xh = np.random.default_rng(6).standard_normal(n)
+    S = capi.System.from_crs(Sw)
+    ref = O.spmv(O.CRS(Sw.rowptr, Sw.colind, Sw.val), xh)
+
+    def call(px, py):
+        assert capi.lib().nlhipSpMV(S._h, C.c_void_p(px), C.c_void_p(py)) == 0
+
+    for xo, yo in ((2, n + 8 & ~1), (3, n + 8 | 1), (2, n + 9 | 1), (3, n + 8 & ~1),
+                   (2, 2), (3, 3), (2, 4), (4, 2), (2, 2 + n)):
+        buf = torch.full((2 * n + 32,), 7.0, dtype=torch.float64, device="cuda")
+        buf[xo:xo + n] = torch.from_numpy(xh).cuda()
+        want = buf.cpu().numpy()
+        want[yo:yo + n] = ref
+        torch.cuda.synchronize()
+        call(buf.data_ptr() + 8 * xo, buf.data_ptr() + 8 * yo)
+        assert np.array_equal(buf.cpu().numpy(), want), (xo, yo)
+    x = torch.from_numpy(xh).cuda()
+    y = torch.zeros_like(x)
+    yh = np.zeros(n)
+    torch.cuda.synchronize()
+    call(xh.ctypes.data, y.data_ptr())
+    assert np.array_equal(y.cpu().numpy(), ref)
+    call(x.data_ptr(), yh.ctypes.data)
+    assert np.array_equal(yh, ref)
+    S.close()
+
+
 def test_spmv_through_opennl_api(hip):
     L = hip
     Sw = W.lscm_grid(20, seed=1)
