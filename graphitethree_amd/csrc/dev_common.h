@@ -122,6 +122,18 @@ __device__ __forceinline__ T ntload(const T* p) {
     return __builtin_nontemporal_load(p);
 }
 
+// Loads and stores that pass the caches (NT) or not.
+template <bool NT, typename T>
+__device__ __forceinline__ T load_as(const T* p) {
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+template <bool NT, typename T>
+__device__ __forceinline__ void store_as(T* p, T v) {
+    if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+
 // Separately rounded multiply and add, so element-wise updates round exactly
 // like a scalar x = x + (a * y) loop.  HIP's __dmul_rn / __dadd_rn are plain
 // operators, so this holds because device code is compiled with

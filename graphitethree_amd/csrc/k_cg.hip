@@ -93,6 +93,34 @@ __global__ __launch_bounds__(kBlock) void k_cg_init_finish(CGArgs<T> a, T eps, i
     }
 }
 
+// Rows [r0, r1) of a direction step: x -= alpha d, d = beta d + h.  Four rows
+// per thread at a time, every load before any store (the arrays may alias as
+// far as the compiler knows).
+template <typename T, bool STREAM_X>
+__device__ __forceinline__ void dir_rows(const CGArgs<T>& a, uint32_t r0, uint32_t r1, T alpha,
+                                         T beta) {
+    uint32_t i = r0 + threadIdx.x;
+    for (; i + 3 * kBlock < r1; i += 4 * kBlock) {
+        T dv[4], xv[4], hv[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            dv[q] = a.d[i + q * kBlock];
+            xv[q] = load_as<STREAM_X>(a.x + i + q * kBlock);
+            hv[q] = a.h[i + q * kBlock];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            store_as<STREAM_X>(a.x + i + q * kBlock, add_rn(xv[q], mul_rn(-alpha, dv[q])));
+            a.d[i + q * kBlock] = add_rn(mul_rn(beta, dv[q]), hv[q]);
+        }
+    }
+    for (; i < r1; i += kBlock) {
+        const T di = a.d[i];
+        a.x[i] = add_rn(a.x[i], mul_rn(-alpha, di));
+        a.d[i] = add_rn(mul_rn(beta, di), a.h[i]);
+    }
+}
+
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_cg_dir(CGArgs<T> a) {
     __shared__ T lds[kWavesPerBlock];
@@ -128,28 +156,8 @@ __global__ __launch_bounds__(kBlock) void k_cg_dir(CGArgs<T> a) {
         for (uint32_t i = r0 + threadIdx.x; i < r1; i += kBlock)
             a.x[i] = add_rn(a.x[i], mul_rn(-alpha, a.d[i]));
     } else {
-        // four rows per thread at a time: every load before any store (the
-        // arrays may alias as far as the compiler knows)
-        uint32_t i = r0 + threadIdx.x;
-        for (; i + 3 * kBlock < r1; i += 4 * kBlock) {
-            T dv[4], xv[4], hv[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                dv[q] = a.d[i + q * kBlock];
-                xv[q] = a.x[i + q * kBlock];
-                hv[q] = a.h[i + q * kBlock];
-            }
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                a.x[i + q * kBlock] = add_rn(xv[q], mul_rn(-alpha, dv[q]));
-                a.d[i + q * kBlock] = add_rn(mul_rn(beta, dv[q]), hv[q]);
-            }
-        }
-        for (; i < r1; i += kBlock) {
-            const T di = a.d[i];
-            a.x[i] = add_rn(a.x[i], mul_rn(-alpha, di));
-            a.d[i] = add_rn(mul_rn(beta, di), a.h[i]);
-        }
+        if (a.streams) dir_rows<T, true>(a, r0, r1, alpha, beta);
+        else dir_rows<T, false>(a, r0, r1, alpha, beta);
     }
 }
 
@@ -179,6 +187,41 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv(CGArgs<T> a) {
     if (threadIdx.x == 0) a.part_dq[L] = pdq;
 }
 
+// Rows [r0, r1) of an update step and the thread's sums of r.h and r.r.  Four
+// rows per thread at a time, loads first; the partial sums take the rows in
+// the same order as one at a time.
+template <typename T, bool PREC, bool STREAM_R, bool STREAM_P>
+__device__ __forceinline__ void update_rows(const CGArgs<T>& a, uint32_t r0, uint32_t r1,
+                                            T alpha, T& prh, T& prr) {
+    uint32_t i = r0 + threadIdx.x;
+    for (; i + 3 * kBlock < r1; i += 4 * kBlock) {
+        T rv[4], qv[4], dv[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            rv[q] = load_as<STREAM_R>(a.r + i + q * kBlock);
+            qv[q] = a.q[i + q * kBlock];
+            dv[q] = PREC ? load_as<STREAM_P>(a.dinv + i + q * kBlock) : T(1);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const T ri = add_rn(rv[q], mul_rn(-alpha, qv[q]));
+            const T hi = PREC ? mul_rn(dv[q], ri) : ri;
+            store_as<STREAM_R>(a.r + i + q * kBlock, ri);
+            a.h[i + q * kBlock] = hi;
+            prh += ri * hi;
+            prr += ri * ri;
+        }
+    }
+    for (; i < r1; i += kBlock) {
+        const T ri = add_rn(a.r[i], mul_rn(-alpha, a.q[i]));
+        const T hi = PREC ? mul_rn(a.dinv[i], ri) : ri;
+        a.r[i] = ri;
+        a.h[i] = hi;
+        prh += ri * hi;
+        prr += ri * ri;
+    }
+}
+
 template <typename T, bool PREC>
 __global__ __launch_bounds__(kBlock) void k_cg_update(CGArgs<T> a) {
     __shared__ T lds[kWavesPerBlock];
@@ -193,35 +236,9 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(CGArgs<T> a) {
     uint32_t r0, r1;
     block_row_range(a.m, a.chunk, L, r0, r1);
     T prh = T(0), prr = T(0);
-    // four rows per thread at a time, loads first; the partial sums take the
-    // rows in the same order as one at a time
-    uint32_t i = r0 + threadIdx.x;
-    for (; i + 3 * kBlock < r1; i += 4 * kBlock) {
-        T rv[4], qv[4], dv[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            rv[q] = a.r[i + q * kBlock];
-            qv[q] = a.q[i + q * kBlock];
-            dv[q] = PREC ? a.dinv[i + q * kBlock] : T(1);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const T ri = add_rn(rv[q], mul_rn(-alpha, qv[q]));
-            const T hi = PREC ? mul_rn(dv[q], ri) : ri;
-            a.r[i + q * kBlock] = ri;
-            a.h[i + q * kBlock] = hi;
-            prh += ri * hi;
-            prr += ri * ri;
-        }
-    }
-    for (; i < r1; i += kBlock) {
-        const T ri = add_rn(a.r[i], mul_rn(-alpha, a.q[i]));
-        const T hi = PREC ? mul_rn(a.dinv[i], ri) : ri;
-        a.r[i] = ri;
-        a.h[i] = hi;
-        prh += ri * hi;
-        prr += ri * ri;
-    }
+    if (a.streams >= 3) update_rows<T, PREC, true, true>(a, r0, r1, alpha, prh, prr);
+    else if (a.streams == 2) update_rows<T, PREC, true, false>(a, r0, r1, alpha, prh, prr);
+    else update_rows<T, PREC, false, false>(a, r0, r1, alpha, prh, prr);
     prh = block_sum_all(prh, lds);
     prr = block_sum_all(prr, lds);
     if (threadIdx.x == 0) {

@@ -140,6 +140,19 @@ hipError_t blas_ddot(uint64_t n, const double* x, const double* y, double* part,
 // out[0] = sum(part[0..P)), out[1] = sqrt(out[0]).
 hipError_t reduce_final(const double* part, uint32_t P, double* out, hipStream_t s);
 
+// Vectors an iteration reads again only after a whole iteration (x, r, dinv)
+// go past the last-level cache, in that order, as far as the six vectors
+// (those, and d, h and q, which the next launch reads) do not all fit it:
+// otherwise they push out d, h and q.  Per 100 iterations on 2x2 block LSCM
+// systems, without -> with: 10.0 M rows (80 MB vectors, three stream) 46.2 ->
+// 43.2 ms, 8.0 M (two) 36.8 -> 35.2, 5.8 M (one) 26.5 -> 25.8, 18 M 84.1 -> 83.8; where all fit, streaming
+// them costs 4% (2.0 M rows: 9.7 -> 10.1 ms).
+constexpr uint64_t kLastLevelCache = 256ull << 20;
+__host__ __device__ inline uint32_t streamed_vectors(uint64_t rows, uint32_t elem) {
+    const uint64_t fit = kLastLevelCache / (rows * elem + 1);
+    return fit >= 6 ? 0u : fit <= 3 ? 3u : uint32_t(6 - fit);
+}
+
 // The SpMV step of the fused PCG runs on up to this many times the
 // workgroups of the other launches (more waves in flight for its gathers).
 constexpr uint32_t kSpmvGridMul = 2;
@@ -153,6 +166,7 @@ struct CGArgs {
     uint32_t P;      // workgroups per launch = number of partial sums
     uint32_t Ps;     // workgroups of the SpMV step (d.q partials), Ps <= kSpmvGridMul P
     uint32_t sps;    // SpMV work per workgroup of the SpMV step
+    uint64_t streams;  // of x, r, dinv: those read and written past the cache
     const uint32_t* rp;
     Cols cols;
     const T* val;

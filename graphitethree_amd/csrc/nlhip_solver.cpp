@@ -248,6 +248,7 @@ void fill_cg_args(const System& S, const CGBuffers<T>& w, const T* dinv, CGArgs<
                               S.grid, std::min<uint64_t>(uint64_t(kSpmvGridMul) * S.grid, quads)))
                         : S.grid;
     a.sps = spmv_work_per_block(S.n, a.Ps, o.code);
+    a.streams = streamed_vectors(S.n, sizeof(T));
     a.rp = o.rp;
     a.cols = o.cols;
     a.val = o.val;

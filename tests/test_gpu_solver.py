@@ -493,3 +493,49 @@ def test_concurrent_solves_from_two_threads(hip):
     [t.join() for t in ts]
     L.nlDeleteMatrix(M)
     assert len(ok) == 10 and all(ok)
+
+
+@pytest.mark.parametrize("n,streams", [(5_592_405 - 5, 0), (5_592_406 + 5, 1),
+                                       (7_000_003, 2), (9_000_001, 3)])
+def test_iterations_whose_vectors_exceed_the_last_level_cache(hip, n, streams):
+    """Around the sizes at which x, r and D^-1 go past the cache one after
+    another: six vectors of 8 n bytes against 256 MiB.  A few iterations on a
+    tridiagonal matrix against a restatement in numpy; the dot products are
+    sums of n positive terms, each off by at most n u, and five iterations
+    form ten of them."""
+    assert max(0, min(3, 6 - (256 << 20) // (8 * n + 1))) == streams
+    rp = np.zeros(n + 1, dtype=np.uint32)
+    rp[1:] = 3
+    rp[1] = rp[n] = 2
+    rp = np.cumsum(rp, dtype=np.uint32)
+    cols = np.arange(n, dtype=np.int64)[:, None] + np.array([-1, 0, 1])
+    keep = (cols >= 0) & (cols < n)
+    rng = np.random.default_rng(n)
+    dia = 2.5 + rng.random(n)
+    val = np.full((n, 3), -1.0)
+    val[:, 1] = dia
+    S = capi.System(rp, cols[keep].astype(np.uint32), val[keep])
+    b = rng.standard_normal(n)
+    x, st = S.solve(b, eps=1e-30, max_iter=5)
+    S.close()
+
+    def mult(v):
+        y = dia * v
+        y[1:] -= v[:-1]
+        y[:-1] -= v[1:]
+        return y
+
+    xr = np.zeros(n)
+    r = -b
+    d = r / dia
+    rho = float(r @ d)
+    for _ in range(5):
+        q = mult(d)
+        alpha = rho / float(d @ q)
+        xr -= alpha * d
+        r -= alpha * q
+        h = r / dia
+        rho, old = float(r @ h), rho
+        d = h + (rho / old) * d
+    assert st.iterations == 5
+    assert rel(x, xr) <= 10 * n * 2.0 ** -53
