@@ -22,15 +22,26 @@ template <int V, typename T>
 struct Lane {
     T v[V];
 };
-template <int V, typename T>
+template <int V, bool NT = false, typename T>
 __device__ __forceinline__ Lane<V, T> lane_load(const T* p) {
     Lane<V, T> r;
-    __builtin_memcpy(r.v, p, sizeof(T) * V);
+    if constexpr (!NT) {
+        __builtin_memcpy(r.v, p, sizeof(T) * V);
+    } else if constexpr (V == 2) {
+        using V2 = T __attribute__((ext_vector_type(2)));
+        const V2 w = __builtin_nontemporal_load(reinterpret_cast<const V2*>(p));
+        r.v[0] = w.x;
+        r.v[1] = w.y;
+    } else {
+        r.v[0] = __builtin_nontemporal_load(p);
+    }
     return r;
 }
-template <int V, typename T>
+template <int V, bool NT = true, typename T>
 __device__ __forceinline__ void lane_store(T* p, const T (&v)[V]) {
-    if constexpr (V == 2) {
+    if constexpr (!NT) {
+        __builtin_memcpy(p, v, sizeof(T) * V);
+    } else if constexpr (V == 2) {
         using V2 = T __attribute__((ext_vector_type(2)));
         V2 w;
         w.x = v[0];

@@ -303,8 +303,19 @@ __global__ __launch_bounds__(kBlock) void k_m_beta(MultiArgs<T> a, int max_iter)
 // before their stores.
 constexpr int kMultiU = 4;
 
+// True when x, d, r and q together exceed the last-level cache: the
+// element-wise steps of larger k then load and store past it (NT), which left
+// it to the rows the SpMM gathers.  Per solve, without -> with: 1500^2 rows x
+// 32 (576 MB each) 8.21 -> 7.87 ms, 1000^2 x 32 (256 MB) 4.04 -> 3.66, 1500^2
+// x 8 (144 MB) 2.48 -> 2.28, 700^2 x 32 (125 MB) 2.05 -> 2.00; the same within
+// 1% at 64 MB and below.
+template <typename T>
+bool multi_streamed(uint32_t m, uint32_t k) {
+    return 4 * uint64_t(m) * k * sizeof(T) > kLastLevelCache;
+}
+
 // Direction step of larger k: V adjacent columns per lane, G / V lanes per row.
-template <int V, typename T, bool PREC>
+template <int V, bool NT, typename T, bool PREC>
 __global__ __launch_bounds__(kBlock) void k_m_dir(MultiArgs<T> a) {
     if (!any_open(a)) return;  // every column has stopped
     const uint32_t L = xcd_logical_block(blockIdx.x, gridDim.x);
@@ -334,9 +345,9 @@ __global__ __launch_bounds__(kBlock) void k_m_dir(MultiArgs<T> a) {
             const uint32_t row = i0 + uint32_t(u) * per;
             if (row < r1) {
                 const uint64_t i = uint64_t(row) * k + j;
-                xv[u] = lane_load<V>(a.x + i);
-                dv[u] = lane_load<V>(a.d + i);
-                rv[u] = lane_load<V>(a.r + i);
+                xv[u] = lane_load<V, NT>(a.x + i);
+                dv[u] = lane_load<V, NT>(a.d + i);
+                rv[u] = lane_load<V, NT>(a.r + i);
                 pv[u] = PREC ? a.dinv[row] : T(1);
             }
         }
@@ -353,8 +364,8 @@ __global__ __launch_bounds__(kBlock) void k_m_dir(MultiArgs<T> a) {
                     xv[u].v[c] = upd[c] ? x : xv[u].v[c];
                     dv[u].v[c] = dir[c] ? d : dv[u].v[c];
                 }
-                __builtin_memcpy(a.x + i, xv[u].v, sizeof(T) * V);
-                __builtin_memcpy(a.d + i, dv[u].v, sizeof(T) * V);
+                lane_store<V, NT>(a.x + i, xv[u].v);
+                lane_store<V, NT>(a.d + i, dv[u].v);
             }
         }
     }
@@ -588,7 +599,7 @@ __global__ __launch_bounds__(kBlock) void k_m_update_few(MultiArgs<T> a) {
 }
 
 // Update step of larger k: V adjacent columns per lane, G / V lanes per row.
-template <int V, typename T, bool PREC>
+template <int V, bool NT, typename T, bool PREC>
 __global__ __launch_bounds__(kBlock) void k_m_update(MultiArgs<T> a) {
     __shared__ T lds[kBlock * V];
     if (!any_active(a)) return;  // every column has stopped (block-uniform)
@@ -616,8 +627,8 @@ __global__ __launch_bounds__(kBlock) void k_m_update(MultiArgs<T> a) {
                 const uint32_t row = i0 + uint32_t(u) * per;
                 if (row < r1) {
                     const uint64_t i = uint64_t(row) * k + j;
-                    rv[u] = lane_load<V>(a.r + i);
-                    qv[u] = lane_load<V>(a.q + i);
+                    rv[u] = lane_load<V, NT>(a.r + i);
+                    qv[u] = lane_load<V, NT>(a.q + i);
                     pv[u] = PREC ? a.dinv[row] : T(1);
                 }
             }
@@ -634,7 +645,7 @@ __global__ __launch_bounds__(kBlock) void k_m_update(MultiArgs<T> a) {
                         prh[c] += ri * hi;
                         prr[c] += ri * ri;
                     }
-                    __builtin_memcpy(a.r + i, rv[u].v, sizeof(T) * V);
+                    lane_store<V, NT>(a.r + i, rv[u].v);
                 }
             }
         }
@@ -927,13 +938,16 @@ static hipError_t multi_iteration_p(const MultiArgs<T>& a, int max_iter, hipStre
     }
     const bool v2 = multi_two_cols<T>(a.k);
     k_m_beta<T><<<a.k, kBlock, 0, s>>>(a, max_iter);
-    if (v2) k_m_dir<2, T, PREC><<<a.P, kBlock, 0, s>>>(a);
-    else k_m_dir<1, T, PREC><<<a.P, kBlock, 0, s>>>(a);
+    const bool nt = multi_streamed<T>(a.m, a.k);
+    if (v2) (nt ? k_m_dir<2, true, T, PREC> : k_m_dir<2, false, T, PREC>)<<<a.P, kBlock, 0, s>>>(a);
+    else (nt ? k_m_dir<1, true, T, PREC> : k_m_dir<1, false, T, PREC>)<<<a.P, kBlock, 0, s>>>(a);
     NLHIP_G_SWITCH(a.G, (v2 ? k_m_spmm<G, two_cols_v<G>(), T><<<a.P, kBlock, 0, s>>>(a)
                            : k_m_spmm<G, 1, T><<<a.P, kBlock, 0, s>>>(a)));
     k_m_alpha<T><<<a.k, kBlock, 0, s>>>(a);
-    if (v2) k_m_update<2, T, PREC><<<a.P, kBlock, 0, s>>>(a);
-    else k_m_update<1, T, PREC><<<a.P, kBlock, 0, s>>>(a);
+    if (v2)
+        (nt ? k_m_update<2, true, T, PREC> : k_m_update<2, false, T, PREC>)<<<a.P, kBlock, 0, s>>>(a);
+    else
+        (nt ? k_m_update<1, true, T, PREC> : k_m_update<1, false, T, PREC>)<<<a.P, kBlock, 0, s>>>(a);
     return hipGetLastError();
 }
 

@@ -250,3 +250,40 @@ def test_row_engine_edges(hip, k, n, deg):
         tol = (n + 4) * 2.0 ** -52 * np.linalg.norm(abs(M) @ abs(X0[j]) + abs(B[j]))
         assert abs(per[j].rel_residual - want) <= tol / np.linalg.norm(B[j]) + 1e-15 * want
     S.close()
+
+
+@pytest.mark.parametrize("k,n", [(5, 1_677_721), (5, 1_677_723), (6, 1_398_103), (31, 270_603),
+                                 (32, 262_145)])
+def test_multi_rhs_vectors_exceed_the_last_level_cache(hip, k, n):
+    """Just at and above 4 x 8 n k = 256 MiB, one and two columns per lane,
+    ragged last rows: three iterations against a restatement in numpy (sums of
+    n positive terms, each off by at most n u; three iterations form six)."""
+    rp = np.full(n + 1, 3, dtype=np.int64)
+    rp[0], rp[1], rp[n] = 0, 2, 2
+    rp = np.cumsum(rp).astype(np.uint32)
+    cols = np.arange(n, dtype=np.int64)[:, None] + np.array([-1, 0, 1])
+    keep = (cols >= 0) & (cols < n)
+    rng = np.random.default_rng(k)
+    dia = 2.5 + rng.random(n)
+    val = np.full((n, 3), -1.0)
+    val[:, 1] = dia
+    S = capi.System(rp, cols[keep].astype(np.uint32), val[keep])
+    B = rng.standard_normal((k, n))
+    X, per, _ = S.solve_multi(B, eps=1e-30, max_iter=3)
+    S.close()
+    for j in (0, k // 2, k - 1):
+        x, r = np.zeros(n), -B[j]
+        d = r / dia
+        rho = float(r @ d)
+        for _ in range(3):
+            q = dia * d
+            q[1:] -= d[:-1]
+            q[:-1] -= d[1:]
+            alpha = rho / float(d @ q)
+            x -= alpha * d
+            r = r - alpha * q
+            h = r / dia
+            rho, old = float(r @ h), rho
+            d = h + (rho / old) * d
+        assert per[j].iterations == 3
+        assert rel(X[j], x) <= 6 * n * 2.0 ** -53
