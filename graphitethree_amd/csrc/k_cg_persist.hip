@@ -27,8 +27,10 @@
 // lock), and every wait is bounded.  A workgroup that gives up sets
 // kPersistFail and leaves; the others then give up at the latest at the
 // barrier before the solver's vectors, partials and status are written,
-// which is complete for all or for none of them.  The caller continues with
-// the three launches from the unchanged state.
+// which is complete for all or for none of them (grid_barrier.h; a wait that
+// is given up between barriers sets the bit before the next one's count can
+// be complete).  The caller continues with the three launches from the
+// unchanged state.
 //
 // LSCM systems, us per iteration, three launches -> this: 1,150 rows 8.2 ->
 // 4.3; 8 k 14.6 -> 5.5; 24 k 14.2 -> 5.7; 60 k 13.7 -> 7.5; 100 k 17.1 -> 8.8;
@@ -50,6 +52,20 @@ template <typename T>
 __device__ __forceinline__ void st_dev(T* p, T v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// A barrier word in device memory (grid_barrier.h).
+struct DeviceWord {
+    uint32_t* p;
+    __device__ __forceinline__ uint32_t load() const { return ld_dev(p); }
+    __device__ __forceinline__ uint32_t add(uint32_t v) const {
+        return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ uint32_t cas(uint32_t expected, uint32_t desired) const {
+        __hip_atomic_compare_exchange_strong(p, &expected, desired, __ATOMIC_RELAXED,
+                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return expected;
+    }
+    __device__ __forceinline__ void pause() const { __builtin_amdgcn_s_sleep(1); }
+};
 // Every store of this wavefront has reached the device's point of coherence.
 __device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
@@ -227,22 +243,9 @@ __global__ __launch_bounds__(MAXT) void k_cg_persist(CGArgs<T> a, CGPersist<T> p
         wait_stores();
         __syncthreads();
         if (threadIdx.x == 0) {
-            const uint32_t old =
-                __hip_atomic_fetch_add(p.bar + kPersistBarPad * (1u + group), 1u,
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (old + 1u == gsize * epoch)
-                __hip_atomic_fetch_add(p.bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const uint32_t target = ngroups * epoch;
-            uint32_t seen = 0;
-            for (uint32_t k = 0; k < kSpinLimit; ++k) {
-                seen = ld_dev(p.bar);
-                if (seen >= target) break;
-                __builtin_amdgcn_s_sleep(1);
-            }
-            if (seen < target)
-                seen = __hip_atomic_fetch_or(p.bar, kPersistFail, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT);
-            s_ok = seen >= target && !(seen & kPersistFail) ? 1u : 0u;
+            const DeviceWord root{p.bar};
+            barrier_arrive(DeviceWord{p.bar + kPersistBarPad * (1u + group)}, root, gsize, epoch);
+            s_ok = barrier_wait(root, ngroups, epoch, kSpinLimit) ? 1u : 0u;
         }
         __syncthreads();
         return s_ok != 0;

@@ -4,6 +4,7 @@
 
 #include <cstdint>
 
+#include "grid_barrier.h"
 #include "nlhip_types.h"
 
 namespace nlhip {
@@ -197,7 +198,6 @@ hipError_t cg_step_part(const CGArgs<T>& a, int rpw, bool precond, int part, hip
 // Many iterations per launch (k_cg_persist.hip) for systems whose matrix fits
 // in registers.
 constexpr uint32_t kPersistBarPad = 32;          // words between barrier counters
-constexpr uint32_t kPersistFail = 0x80000000u;   // bit of bar[0]: a wait was given up
 constexpr int kPersistSmall = 1, kPersistRows = 2, kPersistBlocks = 3;
 template <typename T>
 struct CGPersist {
