@@ -231,6 +231,8 @@ SIGNATURES = {
     "nlhipServerDestroy": (C.c_int, [_vp]),
     "nlhipLastError": (C.c_char_p, []),
     "nlhipInjectFailures": (None, [C.c_int]),
+    "nlhipSystemPersistInfo": (C.c_int, [_vp, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)]),
+    "nlhipSystemSetWaitPolls": (C.c_int, [_vp, C.c_uint32, C.c_uint32]),
     "nlhipDeviceInfo": (C.c_int, [C.c_char_p, C.c_size_t, C.POINTER(C.c_int),
                                   C.POINTER(C.c_uint64)]),
 }
@@ -414,6 +416,17 @@ class System:
         check(lib().nlhipSystemAutotune(self._h, 1 if fp32 else 0, iters, C.byref(rpw),
                                         C.byref(wg), C.byref(t)), "nlhipSystemAutotune")
         return int(rpw.value), int(wg.value), float(t.value)
+
+    def persist_info(self):
+        """(launches of many PCG iterations, those that gave up a wait)."""
+        n, g = C.c_uint64(), C.c_uint64()
+        check(lib().nlhipSystemPersistInfo(self._h, C.byref(n), C.byref(g)), "persist info")
+        return int(n.value), int(g.value)
+
+    def set_wait_polls(self, barrier: int = 0, sums: int = 0):
+        """Test hook: polls after which such a wait is given up (0: default,
+        2^32 - 1: none)."""
+        check(lib().nlhipSystemSetWaitPolls(self._h, barrier, sums), "set wait polls")
 
     def info(self):
         n, nnz, b = C.c_uint32(), C.c_uint64(), C.c_uint64()

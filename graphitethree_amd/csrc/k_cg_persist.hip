@@ -30,7 +30,7 @@
 // which is complete for all or for none of them (grid_barrier.h; a wait that
 // is given up between barriers sets the bit before the next one's count can
 // be complete).  The caller continues with the three launches from the
-// unchanged state.
+// unchanged state, and keeps to them for a while (System::persist).
 //
 // LSCM systems, us per iteration, three launches -> this: 1,150 rows 8.2 ->
 // 4.3; 8 k 14.6 -> 5.5; 24 k 14.2 -> 5.7; 60 k 13.7 -> 7.5; 100 k 17.1 -> 8.8;
@@ -41,8 +41,6 @@
 namespace nlhip {
 
 namespace {
-
-constexpr uint32_t kSpinLimit = 1u << 20;  // polls of one wait (about a second)
 
 template <typename T>
 __device__ __forceinline__ T ld_dev(const T* p) {
@@ -245,7 +243,7 @@ __global__ __launch_bounds__(MAXT) void k_cg_persist(CGArgs<T> a, CGPersist<T> p
         if (threadIdx.x == 0) {
             const DeviceWord root{p.bar};
             barrier_arrive(DeviceWord{p.bar + kPersistBarPad * (1u + group)}, root, gsize, epoch);
-            s_ok = barrier_wait(root, ngroups, epoch, kSpinLimit) ? 1u : 0u;
+            s_ok = barrier_wait(root, ngroups, epoch, p.polls) ? 1u : 0u;
         }
         __syncthreads();
         return s_ok != 0;
@@ -289,7 +287,7 @@ __global__ __launch_bounds__(MAXT) void k_cg_persist(CGArgs<T> a, CGPersist<T> p
                 const uint32_t i = k + uint32_t(lane);
                 T t[N];
                 bool good = false;
-                for (uint32_t polls = 0; !good && polls < kSpinLimit; ++polls) {
+                for (uint32_t polls = 0; !good && polls < p.sum_polls; ++polls) {
                     good = true;
 #pragma unroll
                     for (int q = 0; q < N; ++q) {

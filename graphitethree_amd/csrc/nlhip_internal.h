@@ -4,6 +4,7 @@
 #pragma once
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdint>
 #include <cstring>
@@ -445,6 +446,22 @@ struct PcgOps {
     virtual void norms(double& rr, double& bb) = 0;
 };
 
+// Use of the launches of many iterations on one system.  A launch that gave
+// up a wait (other work holds the compute units) has cost up to about a
+// second, so the next `backoff` runs of iterations keep to the captured
+// launches, twice as many after each further one, until a launch completes.
+struct PersistUse {
+    static constexpr uint32_t kFirst = 16, kMost = 4096;
+    uint32_t polls = kPersistPolls, sum_polls = kPersistPolls;  // per wait
+    uint32_t skip = 0, backoff = 0;
+    uint64_t launches = 0, given_up = 0;
+    void gave_up() {
+        ++given_up;
+        backoff = backoff ? std::min(2 * backoff, kMost) : kFirst;
+        skip = backoff;
+    }
+};
+
 // A CRS matrix resident on the device, with its Jacobi inverse diagonal and
 // (optionally) FP32 copies, its own stream and reusable solve workspaces.
 struct System {
@@ -474,6 +491,7 @@ struct System {
     MultiWork<float> m32;
     DevBuf<double> mscale;
     PcgState pcg;            // the FP64 solve open on ws64 (nlhipSolveBegin)
+    PersistUse persist;
     PinnedBuf<double> host_scalars;
 
     void ensure_fp32();

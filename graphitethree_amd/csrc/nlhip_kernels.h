@@ -198,6 +198,7 @@ hipError_t cg_step_part(const CGArgs<T>& a, int rpw, bool precond, int part, hip
 // Many iterations per launch (k_cg_persist.hip) for systems whose matrix fits
 // in registers.
 constexpr uint32_t kPersistBarPad = 32;          // words between barrier counters
+constexpr uint32_t kPersistPolls = 1u << 20;     // of one wait: about a second
 constexpr int kPersistSmall = 1, kPersistRows = 2, kPersistBlocks = 3;
 template <typename T>
 struct CGPersist {
@@ -206,6 +207,7 @@ struct CGPersist {
     uint32_t stride;   // every stride-th workgroup of the grid does
     uint32_t threads;  // per workgroup
     uint32_t n_iter;   // iterations of this launch
+    uint32_t polls, sum_polls;  // after which a barrier, a sum is given up
     T* dh;             // 2 m: (d, h) of every row
     uint64_t* slots;   // persist_slot_words(P): tagged d.q, r.h and r.r partials
     uint32_t* bar;     // 9 kPersistBarPad words: root counter, one per XCD

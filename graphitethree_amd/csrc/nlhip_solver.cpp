@@ -288,14 +288,20 @@ constexpr uint32_t kPersistIters = 4096;
 // Runs a started CG (arguments set, status open) with many iterations per
 // launch until its loop has stopped (the status in fin).  False where the
 // system is not of that kind, another such kernel holds the device, or a
-// grid-wide wait was given up: the state is then where the captured
-// iterations, which form the same sums, continue.
+// grid-wide wait was given up, now or a short while ago (PersistUse): the
+// state is then where the captured iterations, which form the same sums,
+// continue.
 template <typename T>
 static bool run_persist(System& S, CGWorkspace<T>& ws, CGStatus<T>& fin) {
     if (direct_launches()) return false;
     CGPersist<T> p{};
     cg_persist_plan<T>(ws.args, ws.code, uint32_t(std::max(0, device().cu_count)), p);
     if (!p.kind) return false;
+    PersistUse& use = S.persist;
+    if (use.skip) {
+        --use.skip;
+        return false;
+    }
     std::unique_lock<std::mutex> lock(grid_barrier_mutex(), std::try_to_lock);
     if (!lock.owns_lock()) return false;
     hipStream_t s = S.stream.get();
@@ -304,6 +310,8 @@ static bool run_persist(System& S, CGWorkspace<T>& ws, CGStatus<T>& fin) {
     ws.bar.ensure(9 * kPersistBarPad);
     ws.bar_host.ensure(1);
     p.n_iter = kPersistIters;
+    p.polls = use.polls;
+    p.sum_polls = use.sum_polls;
     p.dh = ws.dh.get();
     p.slots = ws.slots.get();
     p.bar = ws.bar.get();
@@ -313,9 +321,14 @@ static bool run_persist(System& S, CGWorkspace<T>& ws, CGStatus<T>& fin) {
         NLHIP_CHECK(hipMemcpyAsync(host, ws.st.get(), sizeof(CGStatus<T>), hipMemcpyDeviceToHost, s));
         NLHIP_CHECK(hipMemcpyAsync(ws.bar_host.get(), p.bar, 4, hipMemcpyDeviceToHost, s));
         S.stream.sync();
-        if (ws.bar_host.get()[0] & kPersistFail) return false;
+        ++use.launches;
+        if (ws.bar_host.get()[0] & kPersistFail) {
+            use.gave_up();
+            return false;
+        }
         if (host[0].done) break;
     }
+    use.backoff = 0;
     fin = host[0];
     return true;
 }
@@ -1192,6 +1205,28 @@ NLAPI int NLAPIENTRY nlhipSolveAdvance(nlhip_system s, uint32_t iters, int* fini
 
 NLAPI int NLAPIENTRY nlhipSolveEnd(nlhip_system s, double* x, nlhip_solve_stats* stats) {
     return guarded("nlhipSolveEnd", [&] { sliced_end(*sys(s), x, stats); });
+}
+
+NLAPI int NLAPIENTRY nlhipSystemSetWaitPolls(nlhip_system s, uint32_t barrier,
+                                             uint32_t sum) {
+    return guarded("nlhipSystemSetWaitPolls", [&] {
+        System* S = sys(s);
+        std::lock_guard<std::mutex> lock(S->mu);
+        auto limit = [](uint32_t v) { return v == ~0u ? 0u : v ? v : kPersistPolls; };
+        S->persist.polls = limit(barrier);
+        S->persist.sum_polls = limit(sum);
+        S->persist.skip = S->persist.backoff = 0;
+    });
+}
+
+NLAPI int NLAPIENTRY nlhipSystemPersistInfo(nlhip_system s, uint64_t* launches,
+                                            uint64_t* given_up) {
+    return guarded("nlhipSystemPersistInfo", [&] {
+        System* S = sys(s);
+        std::lock_guard<std::mutex> lock(S->mu);
+        if (launches) *launches = S->persist.launches;
+        if (given_up) *given_up = S->persist.given_up;
+    });
 }
 
 NLAPI int NLAPIENTRY nlhipSpMV(nlhip_system s, const double* x, double* y) {

@@ -437,6 +437,16 @@ NLAPI int NLAPIENTRY nlhipServerInfo(nlhip_server s, nlhip_server_info* info);
 NLAPI int NLAPIENTRY nlhipServerDestroy(nlhip_server s);
 
 NLAPI const char* NLAPIENTRY nlhipLastError(void);
+/* Launches of many PCG iterations each that solves of this system have made
+ * (systems of up to a few hundred thousand rows), and how many of them gave up
+ * a grid-wide wait because other work held the device; those solves went on
+ * in launches of one step each, with the same bits.  Either may be null. */
+NLAPI int NLAPIENTRY nlhipSystemPersistInfo(nlhip_system s, uint64_t* launches,
+                                            uint64_t* given_up);
+/* Test hook: polls after which such a wait is given up, at the barriers that
+ * begin and end a launch and for the sums in between (0: the default, about a
+ * second; ~0: no poll, every sum is given up); forgets earlier ones that were. */
+NLAPI int NLAPIENTRY nlhipSystemSetWaitPolls(nlhip_system s, uint32_t barrier, uint32_t sum);
 /* Test hook: the next `count` solves fail with NLHIP_ERR_INJECTED before
  * touching the device (other requests are unaffected). */
 NLAPI void NLAPIENTRY nlhipInjectFailures(int count);

@@ -64,7 +64,7 @@ def cases():
     return c
 
 
-def digests():
+def digests(launches=None):
     capi.lib().nlInitExtension(b"HIP")
     out = {}
     for name, Sw, create, params in cases():
@@ -84,6 +84,8 @@ def digests():
             x, st = S.solve_end()
             rows.append([hashlib.sha256(x.tobytes()).hexdigest(), st.iterations])
             assert rows[-1] == rows[0][:2], name
+        if launches is not None:
+            launches[name] = S.persist_info()
         S.close()
         out[name] = rows
     return out
@@ -96,7 +98,66 @@ def test_same_bits_as_three_launches(hip):
                        env=dict(os.environ, NLHIP_DIRECT_LAUNCH="1"))
     assert r.returncode == 0, r.stderr[-2000:]
     ref = json.loads(r.stdout.split("DIGESTS")[1])
-    got = digests()
+    launches = {}
+    got = digests(launches)
     assert set(got) == set(ref)
     for name in got:
         assert got[name] == ref[name], name
+    # and they are not the three launches: blocks_262146 alone is too large
+    for name, (n, given_up) in launches.items():
+        assert given_up == 0 and (n > 0) == (name != "blocks_262146"), (name, n, given_up)
+
+
+NO_POLLS = 2 ** 32 - 1
+
+
+# one workgroup in eight of the grid, two tiles, four tiles, 2x2 blocks
+@pytest.mark.parametrize("n,pairs", [(4000, False), (20000, False), (65537, False),
+                                     (140002, True)])
+def test_given_up_waits_leave_the_state_to_the_launches(hip, n, pairs):
+    """Waits given up after a few polls, in the first barrier, between steps or
+    not at all: the bits of an undisturbed solve whichever it is, FP64 (whole
+    and in slices) and refined."""
+    Sw = random_spd(n, 6, n, pairs)
+    x0 = np.linspace(-1.0, 1.0, n)
+
+    def solves(S, *polls):
+        S.set_wait_polls(*polls)
+        out = [S.solve(Sw.b, x0=x0, confirm=0)]
+        S.set_wait_polls(*polls)
+        out.append(S.solve(Sw.b, precision="mixed"))
+        S.solve_begin(Sw.b)
+        fin = False
+        while not fin:
+            S.set_wait_polls(*polls)
+            fin, _ = S.solve_advance(5)
+        out.append(S.solve_end())
+        return [(x.tobytes(), st.iterations, st.rel_residual) for x, st in out]
+
+    S = capi.System.from_crs(Sw, fp32=True)
+    want = solves(S)
+    assert S.persist_info()[1] == 0
+    for n_polls in (NO_POLLS, 1, 2, 3, 5, 9, 17, 33, 65, 129, 257, 513, 1025):
+        for polls in ((n_polls, 0), (0, n_polls), (n_polls, n_polls)):
+            n, was = S.persist_info()
+            assert solves(S, *polls) == want, polls
+            if polls == (0, NO_POLLS):  # every launch gives up its first sum
+                assert S.persist_info()[1] - was == S.persist_info()[0] - n > 2
+    S.close()
+
+
+def test_a_given_up_wait_is_not_tried_again_at_once(hip):
+    Sw = random_spd(20000, 6, 3)
+    S = capi.System.from_crs(Sw)
+    S.set_wait_polls(0, NO_POLLS)
+    x, _ = S.solve(Sw.b, confirm=0)
+    assert S.persist_info() == (1, 1)
+    for i in range(16):  # the solves that keep to the launches
+        assert np.array_equal(S.solve(Sw.b, confirm=0)[0], x)
+        assert S.persist_info() == (1, 1), i
+    S.solve(Sw.b, confirm=0)
+    assert S.persist_info() == (2, 2)
+    S.set_wait_polls()  # forgets it
+    assert np.array_equal(S.solve(Sw.b, confirm=0)[0], x)
+    assert S.persist_info() == (3, 2)
+    S.close()
