@@ -23,7 +23,8 @@
 // 9.0 us instead of 4.3).
 //
 // The launch is not cooperative: it uses at most one workgroup of 512 threads
-// per CU, at most one such launch runs at a time in a process (the caller's
+// per CU, which one always holds, at most one such launch runs at a time in a
+// process (the caller's
 // lock), and every wait is bounded.  A workgroup that gives up sets
 // kPersistFail and leaves; the others then give up at the latest at the
 // barrier before the solver's vectors, partials and status are written,
@@ -151,14 +152,14 @@ __global__ __launch_bounds__(MAXT) void k_cg_persist(CGArgs<T> a, CGPersist<T> p
     // (the loop has more scalars than scalar registers; held in registers they
     // cost 0.1 us per iteration)
     __shared__ uint32_t s_polls[2];
-    if (blockIdx.x % p.stride) return;
+    if (blockIdx.x % p.shape.stride) return;
     CGStatus<T>* st = a.st;
     if (st->done) return;  // written by an earlier launch
-    const uint32_t wg = blockIdx.x / p.stride;
-    const uint32_t gw = p.stride > 1 ? wg : xcd_logical_block(wg, p.wgs);
-    const uint32_t group = p.stride > 1 ? 0u : wg % kNumXcd;
-    const uint32_t gsize = p.stride > 1 ? p.wgs : (p.wgs - group + kNumXcd - 1) / kNumXcd;
-    const uint32_t ngroups = p.stride > 1 ? 1u : (p.wgs < kNumXcd ? p.wgs : kNumXcd);
+    const uint32_t wg = blockIdx.x / p.shape.stride, wgs = p.shape.wgs;
+    const uint32_t gw = p.shape.stride > 1 ? wg : xcd_logical_block(wg, wgs);
+    const uint32_t group = p.shape.stride > 1 ? 0u : wg % kNumXcd;
+    const uint32_t gsize = p.shape.stride > 1 ? wgs : (wgs - group + kNumXcd - 1) / kNumXcd;
+    const uint32_t ngroups = p.shape.stride > 1 ? 1u : (wgs < kNumXcd ? wgs : kNumXcd);
     const uint32_t subs = blockDim.x / (64 * AW);
     const uint32_t sub = threadIdx.x / (64 * AW), tid = threadIdx.x % (64 * AW);
     const int lane = threadIdx.x & (kWave - 1);
@@ -510,53 +511,37 @@ __global__ void k_persist_reset(uint32_t* bar, uint64_t* slots, uint32_t words) 
 }
 
 template <typename T>
+static void (*persist_kernel(int kind))(CGArgs<T>, CGPersist<T>) {
+    return kind == kPersistSmall  ? &k_cg_persist<T, false, 2, 1, 512>
+           : kind == kPersistRows ? &k_cg_persist<T, false, 4, 1, 512>
+                                  : &k_cg_persist<T, true, 4, 2, 512>;
+}
+
+template <typename T>
 hipError_t cg_persist(const CGArgs<T>& a, const CGPersist<T>& p, hipStream_t s) {
-    if (a.m == 0 || a.P == 0 || p.wgs == 0 || p.kind == 0) return hipErrorInvalidValue;
-    const uint32_t grid = (p.wgs - 1) * p.stride + 1;
+    const PersistShape& h = p.shape;
+    if (a.m == 0 || a.P == 0 || h.wgs == 0 || h.kind == 0) return hipErrorInvalidValue;
+    const uint32_t grid = (h.wgs - 1) * h.stride + 1;
     k_persist_reset<<<4, kBlock, 0, s>>>(p.bar, p.slots, persist_slot_words<T>(a.P));
-    if (p.kind == kPersistSmall)
-        k_cg_persist<T, false, 2, 1, 512><<<grid, p.threads, 0, s>>>(a, p);
-    else if (p.kind == kPersistRows)
-        k_cg_persist<T, false, 4, 1, 512><<<grid, p.threads, 0, s>>>(a, p);
-    else
-        k_cg_persist<T, true, 4, 2, 512><<<grid, p.threads, 0, s>>>(a, p);
+    persist_kernel<T>(h.kind)<<<grid, h.threads, 0, s>>>(a, p);
     return hipGetLastError();
 }
 template hipError_t cg_persist<double>(const CGArgs<double>&, const CGPersist<double>&,
                                        hipStream_t);
 template hipError_t cg_persist<float>(const CGArgs<float>&, const CGPersist<float>&, hipStream_t);
 
-// The kind of a system's launch, or 0: as many logical
-// workgroups for the SpMV step as for the others, at most one tile per
-// wavefront, one of the engines with contiguous tiles (their twins with
-// other chunk widths or column formats form the same sums).
-//   small  up to 128 rows each, in two wavefronts
-//   rows   up to 256 rows each, at most 2 per CU
-//   blocks up to 512 rows (256 row pairs) each, at most 2 per CU
-// Logical workgroups per physical one: fewer, larger workgroups wait for one
-// another faster until their gathers queue up (us per iteration with 1, 2, 4:
-// 8 k rows 5.6, 5.3, 5.9; 24 k 8.9, 6.0, 5.6; with 1, 2: 100 k 14.9, 9.3).  On
-// one XCD (stride) up to 16 workgroups: 4.0 against 4.3 at 1,150 rows; the
-// gathers of more of them crowd its L2 (8 k rows 7.0 against 5.3).
+// The launch of a system (kind 0: none): as many logical workgroups for the
+// SpMV step as for the others, one of the engines with contiguous tiles
+// (their twins with other chunk widths or column formats form the same sums),
+// and no more workgroups than are resident.
 template <typename T>
 void cg_persist_plan(const CGArgs<T>& a, int code, uint32_t cus, CGPersist<T>& p) {
-    p.kind = 0;
+    p.shape = PersistShape{};
     const bool blk = code >= 73;
     const bool known = (code >= 65 && code <= 68) || code == 71 || code == 72 ||
                        (blk && code <= 79 && code != 77);
-    if (!known || a.Ps != a.P || a.P == 0 || cus < 32) return;
-    uint32_t subs = 2;
-    p.stride = 1;
-    if (!blk && a.sps <= 2 && a.chunk <= 128 && a.P <= 256) {
-        p.kind = kPersistSmall;
-        if (a.P > 128) subs = 4;
-        if (a.P <= 32) p.stride = kNumXcd;
-        p.threads = 128 * subs;
-    } else if (a.sps <= 4 && a.chunk <= (blk ? 512u : 256u) && a.P <= 2 * cus) {
-        p.kind = blk ? kPersistBlocks : kPersistRows;
-        p.threads = 256 * subs;
-    }
-    p.wgs = (a.P + subs - 1) / subs;
+    if (!known || a.Ps != a.P) return;
+    p.shape = persist_resident(persist_shape(blk, a.P, a.sps, a.chunk, kNumXcd), cus, kNumXcd);
 }
 template void cg_persist_plan<double>(const CGArgs<double>&, int, uint32_t, CGPersist<double>&);
 template void cg_persist_plan<float>(const CGArgs<float>&, int, uint32_t, CGPersist<float>&);

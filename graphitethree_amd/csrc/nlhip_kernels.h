@@ -6,6 +6,7 @@
 
 #include "grid_barrier.h"
 #include "nlhip_types.h"
+#include "persist_plan.h"
 
 namespace nlhip {
 
@@ -199,13 +200,9 @@ hipError_t cg_step_part(const CGArgs<T>& a, int rpw, bool precond, int part, hip
 // in registers.
 constexpr uint32_t kPersistBarPad = 32;          // words between barrier counters
 constexpr uint32_t kPersistPolls = 1u << 20;     // of one wait: about a second
-constexpr int kPersistSmall = 1, kPersistRows = 2, kPersistBlocks = 3;
 template <typename T>
 struct CGPersist {
-    int kind;          // 0: not for this system
-    uint32_t wgs;      // workgroups that take part
-    uint32_t stride;   // every stride-th workgroup of the grid does
-    uint32_t threads;  // per workgroup
+    PersistShape shape;
     uint32_t n_iter;   // iterations of this launch
     uint32_t polls, sum_polls;  // after which a barrier, a sum is given up
     T* dh;             // 2 m: (d, h) of every row

@@ -296,7 +296,7 @@ static bool run_persist(System& S, CGWorkspace<T>& ws, CGStatus<T>& fin) {
     if (direct_launches()) return false;
     CGPersist<T> p{};
     cg_persist_plan<T>(ws.args, ws.code, uint32_t(std::max(0, device().cu_count)), p);
-    if (!p.kind) return false;
+    if (!p.shape.kind) return false;
     PersistUse& use = S.persist;
     if (use.skip) {
         --use.skip;

@@ -1,5 +1,6 @@
-"""The give-up protocol of the grid barrier (csrc/grid_barrier.h), every
-access a scheduling point of a model on the host."""
+"""The launches of many PCG iterations, on the host: the give-up protocol of
+their grid barrier (csrc/grid_barrier.h), every access a scheduling point of a
+model, and their choice (csrc/persist_plan.h)."""
 import os
 import subprocess
 
@@ -8,15 +9,19 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-@pytest.fixture(scope="module")
-def barrier(tmp_path_factory):
-    out = str(tmp_path_factory.mktemp("protocol") / "grid_barrier")
+def build(tmp_path_factory, name):
+    out = str(tmp_path_factory.mktemp("protocol") / name)
     r = subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror",
                         "-I" + os.path.join(ROOT, "graphitethree_amd", "csrc"),
-                        os.path.join(ROOT, "tests", "protocol", "grid_barrier.cpp"), "-o", out],
+                        os.path.join(ROOT, "tests", "protocol", name + ".cpp"), "-o", out],
                        stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     assert r.returncode == 0, r.stdout
     return out
+
+
+@pytest.fixture(scope="module")
+def barrier(tmp_path_factory):
+    return build(tmp_path_factory, "grid_barrier")
 
 
 # workgroups, barriers, polls, groups, the one that gives up in between, samples
@@ -33,3 +38,10 @@ def test_all_workgroups_pass_a_barrier_or_none(barrier, n, barriers, polls, grou
     assert total > 0
     assert passed == 0 if quitter >= 0 else passed > 0  # both outcomes are met
     assert n == 1 or passed < total
+
+
+def test_workgroups_that_wait_for_one_another_are_resident(tmp_path_factory):
+    r = subprocess.run([build(tmp_path_factory, "persist_plan")], stdout=subprocess.PIPE,
+                       text=True, timeout=100)
+    assert r.returncode == 0, r.stdout
+    assert int(r.stdout.split()[3]) > 0
