@@ -20,6 +20,7 @@
 namespace nlhip {
 
 constexpr uint32_t kPersistFail = 0x80000000u;  // bit of the root: a wait was given up
+constexpr uint32_t kPersistLong = 0x40000000u;  // with it: by a workgroup whose rows are too long
 
 // Word: load(), add(v) and cas(expected, desired), which returns the value it
 // found, each one atomic access; pause() between polls.

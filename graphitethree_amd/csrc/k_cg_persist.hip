@@ -1,6 +1,6 @@
 // The fused PCG of k_cg.hip with many iterations per launch, for systems
-// whose matrix fits in the registers of the workgroups that are resident at
-// once: below a few hundred thousand rows an iteration of three launches is
+// whose matrix (but for the ends of its longer rows) fits in the registers of
+// the workgroups that are resident at once: below a few hundred thousand rows an iteration of three launches is
 // all latency (14 us for 24 k rows, of which the bytes need one).
 //
 // Every logical workgroup L of the three launches (its 64-row tiles of the
@@ -213,6 +213,14 @@ __global__ __launch_bounds__(MAXT) void k_cg_persist(CGArgs<T> a, CGPersist<T> p
         if (__ballot(jb + uint32_t(u) < je)) most = uint32_t(u) + 1u;
     }
     const uint32_t len = je - jb;
+    // rows for the launches (persist_longest): no state has been written, and
+    // without this workgroup no barrier passes
+    if (__syncthreads_or(len > p.longest)) {
+        if (threadIdx.x == 0)
+            __hip_atomic_fetch_or(p.bar, kPersistFail | kPersistLong, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+        return;
+    }
 
     // the lane's rows of the element-wise steps
     uint32_t r0 = 0, r1 = 0;
@@ -448,7 +456,8 @@ __global__ __launch_bounds__(MAXT) void k_cg_persist(CGArgs<T> a, CGPersist<T> p
                         }
                 }
             }
-            for (uint32_t j = jb + uint32_t(W); j < je; ++j) {  // the rest of a long row
+            // the rest of a longer row, an entry at a time
+            for (uint32_t j = jb + uint32_t(W); j < je; ++j) {
                 const uint32_t cj = NR * kPair * column(j);
                 T v[NV], xv[NR];
                 value(j, v);
@@ -535,15 +544,18 @@ template hipError_t cg_persist<float>(const CGArgs<float>&, const CGPersist<floa
 // (their twins with other chunk widths or column formats form the same sums),
 // and no more workgroups than are resident.
 template <typename T>
-void cg_persist_plan(const CGArgs<T>& a, int code, uint32_t cus, CGPersist<T>& p) {
+void cg_persist_plan(const CGArgs<T>& a, int code, uint64_t nnz, uint32_t cus, CGPersist<T>& p) {
     p.shape = PersistShape{};
     const bool blk = code >= 73;
     const bool known = (code >= 65 && code <= 68) || code == 71 || code == 72 ||
                        (blk && code <= 79 && code != 77);
     if (!known || a.Ps != a.P) return;
     p.shape = persist_resident(persist_shape(blk, a.P, a.sps, a.chunk, kNumXcd), cus, kNumXcd);
+    p.longest = persist_longest(p.shape, nnz, a.m);
 }
-template void cg_persist_plan<double>(const CGArgs<double>&, int, uint32_t, CGPersist<double>&);
-template void cg_persist_plan<float>(const CGArgs<float>&, int, uint32_t, CGPersist<float>&);
+template void cg_persist_plan<double>(const CGArgs<double>&, int, uint64_t, uint32_t,
+                                      CGPersist<double>&);
+template void cg_persist_plan<float>(const CGArgs<float>&, int, uint64_t, uint32_t,
+                                     CGPersist<float>&);
 
 }  // namespace nlhip

@@ -454,6 +454,7 @@ struct PersistUse {
     static constexpr uint32_t kFirst = 16, kMost = 4096;
     uint32_t polls = kPersistPolls, sum_polls = kPersistPolls;  // per wait
     uint32_t skip = 0, backoff = 0;
+    uint32_t long_rows = 0;  // bit per kind: the launch found longer rows than it takes
     uint64_t launches = 0, given_up = 0;
     void gave_up() {
         ++given_up;

@@ -203,6 +203,7 @@ constexpr uint32_t kPersistPolls = 1u << 20;     // of one wait: about a second
 template <typename T>
 struct CGPersist {
     PersistShape shape;
+    uint32_t longest;  // entries of a row (blocks of a row pair) it takes
     uint32_t n_iter;   // iterations of this launch
     uint32_t polls, sum_polls;  // after which a barrier, a sum is given up
     T* dh;             // 2 m: (d, h) of every row
@@ -214,7 +215,7 @@ constexpr uint32_t persist_slot_words(uint32_t P) {
     return 3u * P * uint32_t(sizeof(T) / 4);
 }
 template <typename T>
-void cg_persist_plan(const CGArgs<T>& a, int code, uint32_t cus, CGPersist<T>& p);
+void cg_persist_plan(const CGArgs<T>& a, int code, uint64_t nnz, uint32_t cus, CGPersist<T>& p);
 template <typename T>
 hipError_t cg_persist(const CGArgs<T>& a, const CGPersist<T>& p, hipStream_t s);
 

@@ -287,17 +287,18 @@ constexpr uint32_t kPersistIters = 4096;
 
 // Runs a started CG (arguments set, status open) with many iterations per
 // launch until its loop has stopped (the status in fin).  False where the
-// system is not of that kind, another such kernel holds the device, or a
-// grid-wide wait was given up, now or a short while ago (PersistUse): the
+// system is not of that kind (the first launch looks at its rows), another
+// such kernel holds the device, or a grid-wide wait was given up, now or a short while ago (PersistUse): the
 // state is then where the captured iterations, which form the same sums,
 // continue.
 template <typename T>
 static bool run_persist(System& S, CGWorkspace<T>& ws, CGStatus<T>& fin) {
     if (direct_launches()) return false;
     CGPersist<T> p{};
-    cg_persist_plan<T>(ws.args, ws.code, uint32_t(std::max(0, device().cu_count)), p);
-    if (!p.shape.kind) return false;
+    cg_persist_plan<T>(ws.args, ws.code, S.nnz, uint32_t(std::max(0, device().cu_count)), p);
     PersistUse& use = S.persist;
+    const uint32_t kind_bit = 1u << p.shape.kind;
+    if (!p.shape.kind || (use.long_rows & kind_bit)) return false;
     if (use.skip) {
         --use.skip;
         return false;
@@ -322,6 +323,10 @@ static bool run_persist(System& S, CGWorkspace<T>& ws, CGStatus<T>& fin) {
         NLHIP_CHECK(hipMemcpyAsync(ws.bar_host.get(), p.bar, 4, hipMemcpyDeviceToHost, s));
         S.stream.sync();
         ++use.launches;
+        if (ws.bar_host.get()[0] & kPersistLong) {
+            use.long_rows |= kind_bit;
+            return false;
+        }
         if (ws.bar_host.get()[0] & kPersistFail) {
             use.gave_up();
             return false;

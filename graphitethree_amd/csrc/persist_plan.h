@@ -53,4 +53,25 @@ inline PersistShape persist_resident(PersistShape s, uint32_t cus, uint32_t num_
     return s;
 }
 
+// Entries (2x2 blocks) of the longest row (row pair) it takes: 16 (8) are in
+// registers, and the rest of a row is fetched by its lane one after another in
+// every iteration, 0.2 to 0.3 us each, while everyone waits.  The launches
+// lose little to one long row (their tiles' entries are read side by side), but
+// few workgroups, as small systems have, take long to stream long rows.
+// us per iteration, three launches against this:
+//   24 k rows, one of 41 entries among 5: 12.8, 12.0; of 53 13.0, 14.4; of 505
+//   20.4, 149; all of 49 22.9, 20.9, of 65 27.4, 31.0
+//   8 k, all of 49 22.9, 14.9, of 257 179, 77.5; 1 k, one of 53 14.3, 11.2, of
+//   101 15.3, 21.6, all of 257 186, 76.5
+//   100 k, one of 41 15.2, 14.0, of 53 15.6, 16.5; all of 21 19.8, 12.3, of 25
+//   21.7, 17.5, of 33 23.8, 28.5
+//   100 k pairs, one of 37 blocks 19.6, 18.1, of 69 20.7, 26.3; all of 11 22.5,
+//   18.1, of 13 24.2, 24.3
+inline uint32_t persist_longest(const PersistShape& s, uint64_t nnz, uint32_t n) {
+    const uint32_t mean = uint32_t((nnz + n - 1) / n);  // entries of a row
+    if (s.kind == kPersistSmall) return 40 + (s.threads <= 256 ? mean : mean / 4);
+    if (mean <= 16) return 40;
+    return s.kind == kPersistBlocks ? 12 : 24;
+}
+
 }  // namespace nlhip
