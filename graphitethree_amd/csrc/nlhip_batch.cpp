@@ -159,9 +159,11 @@ void batch_loop(Batch& B, BatchWork<T>& w, bool precond, int max_iter, uint32_t 
         return k;
     };
     uint32_t pgrid = 0;
+    // while another kernel with grid-wide barriers holds the device: in
+    // launches, the same bits
     std::unique_lock<std::mutex> barrier_lock(grid_barrier_mutex(), std::defer_lock);
-    if (B.persistent) {
-        barrier_lock.lock();
+    const bool persistent = B.persistent && barrier_lock.try_lock();
+    if (persistent) {
         NLHIP_CHECK(batch_persistent_grid<T>(w.args, precond, &pgrid));
         pgrid = std::min(pgrid, std::max(B.grid, 1u));
     } else {
@@ -183,7 +185,7 @@ void batch_loop(Batch& B, BatchWork<T>& w, bool precond, int max_iter, uint32_t 
     uint64_t launched = 0, covered = 0;
     for (;;) {
         const uint32_t its = run_len(launched);
-        if (B.persistent) {
+        if (persistent) {
             NLHIP_CHECK(batch_persistent<T>(w.args, precond, max_iter, its, pgrid, s));
         } else if (B.graphs) {
             w.graph.launch(launched, s);

@@ -349,7 +349,8 @@ NLAPI int NLAPIENTRY nlhipBatchSetGraphs(nlhip_batch b, int on);
  * direction, SpMV and update phases separated by grid-wide barriers instead
  * of kernel boundaries, on as many workgroups as the device holds at once
  * (at most the batch's workgroup count).  Same kernels' arithmetic, same
- * bits as the three-launch path; on = 0 (default): captured graphs of three
+ * bits as the three-launch path, which it takes while another solve's kernel
+ * of that sort runs in the process; on = 0 (default): captured graphs of three
  * launches per iteration. */
 NLAPI int NLAPIENTRY nlhipBatchSetPersistent(nlhip_batch b, int on);
 /* Workgroups of the grid that walks the active tiles. */

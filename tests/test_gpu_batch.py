@@ -147,6 +147,40 @@ def test_batch_persistent_launch_gives_the_same_bits(hip, small_atlas):
     B.close()
 
 
+def test_persistent_batch_does_not_wait_for_a_solve(hip, small_atlas):
+    """Kernels with grid-wide barriers run one at a time in a process.  While
+    a long solve holds the device with one, a persistent batch goes on in
+    launches: done before that solve, with the same bits."""
+    import threading
+    import time
+
+    A = small_atlas
+    B = capi.Batch([A.chart(c) for c in range(A.count)])
+    want, _, _ = B.solve(A.b, eps=1e-6, max_iter=100)
+    B.set_persistent(True)
+    B.solve(A.b, eps=1e-6, max_iter=100)
+    Sw = W.lscm_system(W.chart_mesh(12011, 3))
+    S = capi.System.from_crs(Sw)
+    end = {}
+
+    def long_solve():
+        S.solve(Sw.b, eps=1e-140, max_iter=300000, confirm=0)
+        end["solve"] = time.perf_counter()
+
+    t = threading.Thread(target=long_solve)
+    t0 = time.perf_counter()
+    t.start()
+    time.sleep(0.02)
+    got, _, _ = B.solve(A.b, eps=1e-6, max_iter=100)
+    end["batch"] = time.perf_counter()
+    t.join()
+    assert S.persist_info()[0] >= 4  # of 4096 iterations each
+    assert np.array_equal(want.view(np.uint64), got.view(np.uint64))
+    assert end["batch"] < end["solve"], {k: v - t0 for k, v in end.items()}
+    S.close()
+    B.close()
+
+
 def test_batch_launch_shape_does_not_change_bits(hip, small_atlas):
     A = small_atlas
     B = capi.Batch([A.chart(c) for c in range(A.count)])
