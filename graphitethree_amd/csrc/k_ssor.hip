@@ -82,18 +82,30 @@ __global__ __launch_bounds__(kBlock) void k_ssor_sweep(SsorArgs a, uint32_t l) {
 // A run of levels, positions [k0, k1), by one workgroup, level after level.
 //
 // What bounds it is the chain from level to level.  The results of the last
-// kRing positions stay in LDS, where the next level's rows read them (by
-// position, sw.dep; older ones, and those of earlier launches, from memory);
-// everything else a row needs is known before: its packed entries, diagonal
+// kRing - kChain positions are read from LDS, by position (sw.dep); older ones,
+// and those of earlier launches, are known when their chunk begins and are
+// read from memory then, the product taking the place of the entry.
+// Everything else a row needs is known before: its packed entries, diagonal
 // and input are loaded into registers a chunk of kChain positions ahead, the
 // row numbers that lead to them another chunk ahead.  A level then costs LDS
 // reads, the sums, a division and a barrier: 0.73 us against 1.9 with the values
 // through memory (599 levels of up to 300 rows, 300^2 grid: 431 and 518 us a
 // sweep).  What must not stand in the level loop is a load or its wait (1.1
-// us a level), nor a branch per entry (1.0).  512 threads: 485 and 577 us.
+// us a level), nor a branch per entry (1.0): rows of more than kChainE entries
+// take one in the chunks that have them, in groups of kChainX (entry by entry,
+// and every value of such a chunk by a search for it, a level cost 3.5 us).
+// 512 threads: 485 and 577 us.
+//
+// us per application, levels of up to 256 rows through memory in one workgroup
+// and the others over the grid -> this: 300^2 cotangent 2970 -> 1630, 1000^2 14300 ->
+// 10600, 317^2 LSCM 5240 -> 3060, 27-point stencil on 30^3 1080 -> 930 and on 64^3
+// 4340 -> 4180, Delaunay mesh of 200 k vertices numbered by rows 6080 -> 3420, at
+// random 360 -> 360.
 constexpr uint32_t kChain = 1024;   // threads, positions per chunk
 constexpr uint32_t kRing = 16384;   // results kept in LDS (128 KiB)
 constexpr int kChainE = 8;          // entries of a row kept in registers
+constexpr int kChainX = 4;          // of the others, at a time
+constexpr uint32_t kKnown = ~0u;    // dep of an entry kept as its product
 
 struct ChainRow {
     uint32_t row, e0, e1, lev;
@@ -106,11 +118,14 @@ struct ChainData {
 template <bool UPPER>
 __global__ __launch_bounds__(kChain) void k_ssor_chain(SsorArgs a, uint32_t k0, uint32_t k1) {
     extern __shared__ double ring[];
-    __shared__ uint32_t s_lev[2], s_kind[2][2];  // longer than 4 entries, odd
+    // a row of the chunk has more than 4, more than kChainE entries, a value
+    // that is not in the ring
+    __shared__ uint32_t s_lev[2], s_kind[2][3];
     const SsorSweepArgs& sw = UPPER ? a.up : a.lo;
     double* const out = UPPER ? a.y : a.w;
-    // position q's value, as position k reads it
-    auto in_ring = [&](uint32_t q, uint32_t k) { return q >= k0 && k - q <= kRing / 2; };
+    // whether position k reads q's value in LDS (no position of k's chunk has
+    // taken its place)
+    auto in_ring = [&](uint32_t q, uint32_t k) { return q >= k0 && k - q <= kRing - kChain; };
     auto stored = [&](uint32_t q) {
         return __hip_atomic_load(out + sw.rows[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
@@ -143,7 +158,7 @@ __global__ __launch_bounds__(kChain) void k_ssor_chain(SsorArgs a, uint32_t k0, 
     ChainRow r = row_of(k), rn = row_of(k + kChain);
     ChainData c = data_of(k, r);
     uint32_t chunk = 0;
-    if (threadIdx.x < 4) s_kind[threadIdx.x / 2][threadIdx.x % 2] = 0;
+    if (threadIdx.x < 6) s_kind[threadIdx.x / 3][threadIdx.x % 3] = 0;
     __syncthreads();
     for (uint32_t c0 = k0; c0 < k1; c0 += kChain, k += kChain, ++chunk) {
         // this chunk's registers, loaded a chunk ago: used here, so that the
@@ -158,20 +173,39 @@ __global__ __launch_bounds__(kChain) void k_ssor_chain(SsorArgs a, uint32_t k0, 
         const uint32_t len = r.e1 - r.e0;
         if (threadIdx.x == 0) s_lev[0] = r.lev;
         if (threadIdx.x == last) s_lev[1] = r.lev;
-        // an entry that is not kept, or whose value is not in the ring
-        bool odd = len > uint32_t(kChainE);
+        // Values that are not in the ring are known: read here, and kept as
+        // the entry's product.  They are kRing - kChain positions back, in an
+        // earlier group of four chunks, whose stores have been waited for.
+        bool far = false;
 #pragma unroll
         for (int u = 0; u < kChainE; ++u)
-            odd |= k < k1 && uint32_t(u) < len && !in_ring(c.dep[u], k);
-        if (odd) s_kind[chunk & 1u][1] = 1;
+            far |= k < k1 && uint32_t(u) < len && !in_ring(c.dep[u], k);
+        if (far) {
+#pragma unroll
+            for (int u0 = 0; u0 < kChainE; u0 += kChainX) {
+                double g[kChainX];
+#pragma unroll
+                for (int u = u0; u < u0 + kChainX; ++u) {
+                    g[u - u0] = 0.0;
+                    if (uint32_t(u) < len && !in_ring(c.dep[u], k)) g[u - u0] = stored(c.dep[u]);
+                }
+#pragma unroll
+                for (int u = u0; u < u0 + kChainX; ++u)
+                    if (uint32_t(u) < len && !in_ring(c.dep[u], k)) {
+                        c.v[u] = mul_rn(c.v[u], g[u - u0]);
+                        c.dep[u] = kKnown;
+                    }
+            }
+            s_kind[chunk & 1u][2] = 1;
+        }
         if (len > 4u) s_kind[chunk & 1u][0] = 1;
-        // results that are not in the ring are read from memory: kRing / 2
-        // positions back, in an earlier group of four chunks
+        if (len > uint32_t(kChainE)) s_kind[chunk & 1u][1] = 1;
         if (chunk % 4 == 3) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         const uint32_t l0 = s_lev[0], l1 = s_lev[1];
-        const int kind = s_kind[chunk & 1u][1] ? 2 : int(s_kind[chunk & 1u][0]);
-        if (threadIdx.x < 2) s_kind[(chunk + 1u) & 1u][threadIdx.x] = 0;
+        const uint32_t more = s_kind[chunk & 1u][0], most = s_kind[chunk & 1u][1],
+                       known = s_kind[chunk & 1u][2];
+        if (threadIdx.x < 3) s_kind[(chunk + 1u) & 1u][threadIdx.x] = 0;
         const ChainRow rnn = row_of(k + 2 * kChain);
         const ChainData cn = data_of(k + kChain, rn);
         auto finish = [&](double S) {
@@ -179,41 +213,73 @@ __global__ __launch_bounds__(kChain) void k_ssor_chain(SsorArgs a, uint32_t k0, 
             ring[k % kRing] = t;
             out[r.row] = t;
         };
-        // no loads in here: the next chunk's stay in flight.  Past a row's end
-        // a value that is not used.
-        auto levels = [&](auto n) {
+        // the sum of the first N entries; past the row's end a value that is
+        // not used
+        auto kept = [&](auto n, auto pre) {
             constexpr int N = decltype(n)::value;
+            double S = 0.0, g[N];
+#pragma unroll
+            for (int u = 0; u < N; ++u) g[u] = ring[c.dep[u] % kRing];
+#pragma unroll
+            for (int u = 0; u < N; ++u) {
+                double t = mul_rn(c.v[u], g[u]);
+                if (decltype(pre)::value && c.dep[u] == kKnown) t = c.v[u];
+                t = add_rn(S, t);
+                S = uint32_t(u) < len ? t : S;
+            }
+            return S;
+        };
+        // no loads in here: the next chunk's stay in flight
+        auto levels = [&](auto n, auto pre) {
             for (uint32_t l = l0; l <= l1; ++l) {
-                if (k < k1 && r.lev == l) {
-                    double S = 0.0, g[N];
-#pragma unroll
-                    for (int u = 0; u < N; ++u) g[u] = ring[c.dep[u] % kRing];
-#pragma unroll
-                    for (int u = 0; u < N; ++u) {
-                        const double t = add_rn(S, mul_rn(c.v[u], g[u]));
-                        S = uint32_t(u) < len ? t : S;
-                    }
-                    finish(S);
-                }
+                if (k < k1 && r.lev == l) finish(kept(n, pre));
                 __syncthreads();
             }
         };
-        if (kind == 0) {
-            levels(std::integral_constant<int, 4>{});
-        } else if (kind == 1) {
-            levels(std::integral_constant<int, kChainE>{});
-        } else {
+        using N4 = std::integral_constant<int, 4>;
+        using N8 = std::integral_constant<int, kChainE>;
+        if (most) {
+            // the entries past those kept: as many at a time, loads first
+            const bool longer = __any(k < k1 && len > uint32_t(kChainE));
             for (uint32_t l = l0; l <= l1; ++l) {
                 if (k < k1 && r.lev == l) {
-                    double S = 0.0;
-                    for (uint32_t e = r.e0; e < r.e1; ++e) {
-                        const uint32_t q = sw.dep[e];
-                        S = add_rn(S, mul_rn(sw.val[e], in_ring(q, k) ? ring[q % kRing] : stored(q)));
+                    double S = kept(N8{}, std::true_type{});
+                    if (longer) {
+                        for (uint32_t e = r.e0 + kChainE; e < r.e1; e += kChainX) {
+                            uint32_t q[kChainX];
+                            double v[kChainX], g[kChainX];
+                            bool out = false;
+#pragma unroll
+                            for (int u = 0; u < kChainX; ++u) {
+                                const uint32_t at = e + u < r.e1 ? e + u : r.e1 - 1u;
+                                q[u] = sw.dep[at];
+                                v[u] = sw.val[at];
+                            }
+#pragma unroll
+                            for (int u = 0; u < kChainX; ++u) {
+                                g[u] = ring[q[u] % kRing];
+                                out |= !in_ring(q[u], k);
+                            }
+                            if (out) {
+#pragma unroll
+                                for (int u = 0; u < kChainX; ++u)
+                                    if (!in_ring(q[u], k)) g[u] = stored(q[u]);
+                            }
+#pragma unroll
+                            for (int u = 0; u < kChainX; ++u)
+                                if (e + uint32_t(u) < r.e1) S = add_rn(S, mul_rn(v[u], g[u]));
+                        }
                     }
                     finish(S);
                 }
                 __syncthreads();
             }
+        } else if (known) {
+            levels(N8{}, std::true_type{});
+        } else if (more) {
+            levels(N8{}, std::false_type{});
+        } else {
+            levels(N4{}, std::false_type{});
         }
         r = rn;
         rn = rnn;

@@ -12,9 +12,16 @@ namespace nlhip {
 
 namespace {
 
-// Levels of at most this many rows run back to back in one workgroup: 1024 rows
-// take some 0.7 us, and a launch of its own about 3.
-constexpr uint32_t kChainRows = 4096;
+// Levels of at most this many loads (six per row and two per entry it reads)
+// run back to back in one workgroup, larger ones are launches of their own: a
+// launch takes about 4 us, and the one CU of the chain issues a wavefront's
+// loads, which are not coalesced, in some 30 ns each.  us per application with
+// limits of 2500, 5000, 9000, 16000, 24000: 300^2 cotangent 2470, 1630, 1630, 1610,
+// 1620; 317^2 LSCM 5920, 4200, 3060, 3030, 3050; 27-point stencil on 64^3 4360,
+// 4280, 4180, 4200, 4600; 7-point 1500, 1430, 1400, 1470, 1680; Delaunay mesh of
+// 20 k vertices numbered at random 170, 172, 174, 179, 221.  With a limit of 4096
+// rows instead the last three took 9750, 2950 and 350.
+constexpr uint64_t kChainLoads = 9000;
 
 // level(i) = 1 + the deepest level among the rows i reads (j < i for the
 // forward sweep, j > i for the backward one); rows counting-sorted by level
@@ -57,6 +64,7 @@ class Ssor {
   public:
     struct Step {
         uint32_t l0, l1, k0, k1;  // levels [l0, l1), positions [k0, k1)
+        bool grid;                // one level over the whole grid, or a chain
     };
     uint32_t n = 0;
     double omega = 1.5;
@@ -85,25 +93,22 @@ class Ssor {
 
 namespace {
 
-// A level of more than kChainRows rows: over the whole grid.
-bool wide(const Ssor::Step& st) { return st.l1 - st.l0 == 1 && st.k1 - st.k0 > kChainRows; }
-
-// One launch per level with more than kChainRows rows, one workgroup per run
-// of consecutive smaller levels.
-std::vector<Ssor::Step> plan(const std::vector<uint32_t>& off) {
+// One launch per level that is too large for one workgroup, one workgroup
+// per run of consecutive others.  off: first position of each level, eoff:
+// first entry of each position.
+std::vector<Ssor::Step> plan(const std::vector<uint32_t>& off, const std::vector<uint32_t>& eoff) {
     std::vector<Ssor::Step> steps;
     const uint32_t nl = uint32_t(off.size() - 1);
+    auto large = [&](uint32_t l) {
+        const uint64_t rows = off[l + 1] - off[l], entries = eoff[off[l + 1]] - eoff[off[l]];
+        return 6 * rows + 2 * entries > kChainLoads;
+    };
     uint32_t l = 0;
     while (l < nl) {
-        const uint32_t sz = off[l + 1] - off[l];
-        if (sz > kChainRows) {
-            steps.push_back({l, l + 1, off[l], off[l + 1]});
-            ++l;
-            continue;
-        }
-        uint32_t e = l;
-        while (e < nl && off[e + 1] - off[e] <= kChainRows) ++e;
-        steps.push_back({l, e, off[l], off[e]});
+        uint32_t e = l + 1;
+        const bool grid = large(l);
+        while (!grid && e < nl && !large(e)) ++e;
+        steps.push_back({l, e, off[l], off[e], grid});
         l = e;
     }
     return steps;
@@ -120,11 +125,18 @@ std::vector<Ssor::Step> build_sweep(uint32_t n, const std::vector<uint32_t>& rp,
                                     bool upper, SweepBufs& B, hipStream_t s) {
     std::vector<uint32_t> rows, off;
     level_schedule(n, rp, ci, upper, rows, off);
-    std::vector<Ssor::Step> steps = plan(off);
+    std::vector<uint32_t> eoff(size_t(n) + 1, 0);
+    for (uint32_t k = 0; k < n; ++k) {
+        const uint32_t i = rows[k];
+        uint32_t m = 0;
+        for (uint32_t e = rp[i]; e < rp[i + 1]; ++e) m += (upper ? ci[e] > i : ci[e] < i) ? 1u : 0u;
+        eoff[k + 1] = eoff[k] + m;
+    }
+    std::vector<Ssor::Step> steps = plan(off, eoff);
     // columns for the levels launched over the grid, positions for the others
     bool by_col = false, by_pos = false;
-    for (const Ssor::Step& st : steps) (wide(st) ? by_col : by_pos) = true;
-    std::vector<uint32_t> eoff(size_t(n) + 1, 0), col, dep, lev(by_pos ? n : 0), at(by_pos ? n : 0);
+    for (const Ssor::Step& st : steps) (st.grid ? by_col : by_pos) = true;
+    std::vector<uint32_t> col, dep, lev(by_pos ? n : 0), at(by_pos ? n : 0);
     std::vector<double> val;
     val.reserve(ci.size() / 2 + 1);
     if (by_col) col.reserve(ci.size() / 2 + 1);
@@ -142,7 +154,6 @@ std::vector<Ssor::Step> build_sweep(uint32_t n, const std::vector<uint32_t>& rp,
                 if (by_pos) dep.push_back(at[ci[e]]);
                 val.push_back(va[e]);
             }
-        eoff[k + 1] = uint32_t(val.size());
     }
     auto put = [&](auto& dst, const auto& src) {
         if (src.empty()) return;
@@ -202,7 +213,7 @@ Ssor* ssor_create(System& S, double omega) {
     P->graph.capture(s, [&] {
         auto sweep = [&](const std::vector<Ssor::Step>& steps, bool upper) {
             for (const Ssor::Step& st : steps) {
-                if (wide(st))
+                if (st.grid)
                     NLHIP_CHECK(ssor_level(a, upper, st.l0, st.k1 - st.k0, s));
                 else
                     NLHIP_CHECK(ssor_chain(a, upper, st.k0, st.k1, s));

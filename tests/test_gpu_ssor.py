@@ -223,6 +223,9 @@ def chain_patterns():
         c = np.concatenate(lists).astype(np.int64)
         return dominant(sp.coo_matrix((rng.standard_normal(len(r)), (r, c)), shape=(n, n)))
 
+    def both(A):  # the same reads in the backward sweep
+        return (A + A.T).tocsr()
+
     n = 20000
     arrow = rows(n, [np.array([i % 7, max(i - 1, 0), min(i + 1, n - 1), n - 1 - i % 5])
                      for i in range(n)])
@@ -239,14 +242,24 @@ def chain_patterns():
         if i >= 7500:
             mixed[i, 1500 + (i * 7) % 6000] = 0.25
             mixed[i, i % 1000] = -0.5
-    return {"arrow": arrow, "wide_5000": dominant(wide), "long_rows": long,
+    # positions are row numbers: values at and about the end of the ring, among
+    # the first eight entries of a row and past them, and levels of 300 rows
+    # that read others of every age
+    ends = [15359, 15360, 15361, 15362]
+    far = [np.unique(np.concatenate([[i], [max(i - 1, 0)], [i - d for d in ends if d <= i],
+                                     i - rng.integers(1, 40, i % 17) if i > 40 else [i]]))
+           for i in range(n)]
+    aged = [np.unique(np.concatenate([[i], [max(i - 300, 0)], rng.integers(0, i // 300 * 300 + 1,
+                                                                          1 + i % 14)]))
+            for i in range(30000)]
+    return {"arrow": arrow, "ring_ends": both(rows(n, far)), "aged": both(rows(30000, aged)), "wide_5000": dominant(wide), "long_rows": long,
             "mixed": dominant(mixed + mixed.T), "one": sp.identity(1, format="csr") * 3.0,
             "levels_1025": dominant(sp.kron(sp.csr_matrix(np.tri(9) + np.tri(9).T),
                                             sp.eye(1025)))}
 
 
 @pytest.mark.parametrize("name", ["arrow", "wide_5000", "long_rows", "mixed", "one",
-                                  "levels_1025"])
+                                  "levels_1025", "ring_ends", "aged"])
 def test_chain_edges_are_bitwise_the_oracle(hip, name):
     """The one-workgroup run of levels: values that have left the LDS ring or
     come from an earlier launch, levels wider than a chunk, rows of more
