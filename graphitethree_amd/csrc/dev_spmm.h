@@ -17,7 +17,13 @@ __device__ __forceinline__ void spmm_xcd_rows(uint32_t m, uint32_t lo, uint32_t 
 
 // A lane's V adjacent columns of an interleaved vector (V = 2: an aligned
 // pair), loaded and stored as one word.  Stores are non-temporal: the result
-// must not push the gathered rows out of the L2.
+// must not push the gathered rows out of the L2.  At every size: with plain
+// stores the eigensolver is as fast where its blocks fit the last-level cache
+// (88.0 and 88.3 ms at 300^2, 477 and 476 at 500^2) and slower beyond it (925
+// and 963 ms at 600^2, 6.18 and 6.35 s at 1000^2), the multi-RHS iteration
+// between 5% faster and 2.5% slower without a pattern (us, non-temporal and plain:
+// 300^2 x 32 76 and 77, 500^2 x 32 154 and 158, 700^2 x 32 287 and 275, 1000^2 x 32
+// 559 and 571, 1500^2 x 32 1281 and 1299).
 template <int V, typename T>
 struct Lane {
     T v[V];

@@ -204,12 +204,9 @@ __global__ void k_ls_scatter(uint64_t nent, const uint32_t* var, const uint32_t*
     }
 }
 
-__device__ __forceinline__ uint32_t lane_u32(uint32_t v, int l) {
-    return uint32_t(__builtin_amdgcn_readlane(int(v), l));
-}
 __device__ __forceinline__ double lane_f64(double v, int l) {
     const long long b = __double_as_longlong(v);
-    const uint32_t lo = lane_u32(uint32_t(b), l), hi = lane_u32(uint32_t(b >> 32), l);
+    const uint32_t lo = lane_word(uint32_t(b), l), hi = lane_word(uint32_t(b >> 32), l);
     return __longlong_as_double((long long)((uint64_t(hi) << 32) | lo));
 }
 
@@ -243,7 +240,7 @@ __global__ __launch_bounds__(kBlock) void k_ls_wave(
         const uint32_t o0 = occ_off[f], m = occ_off[f + 1] - o0;
         uint32_t k = uint32_t(lane) < m ? occ[o0 + uint32_t(lane)] : kNone;
         uint32_t rank = 0;
-        for (uint32_t i = 0; i < m; ++i) rank += lane_u32(k, int(i)) < k ? 1u : 0u;
+        for (uint32_t i = 0; i < m; ++i) rank += lane_word(k, int(i)) < k ? 1u : 0u;
         // push lane l's entry to lane rank (a permutation of the first m lanes;
         // the others keep their place)
         if (uint32_t(lane) >= m) rank = uint32_t(lane);
@@ -270,7 +267,7 @@ __global__ __launch_bounds__(kBlock) void k_ls_wave(
             uint64_t left = __ballot(f2 != kNone);
             uint64_t todo = 0;  // contributions of this chunk to the owned entry
             while (left) {
-                const uint32_t c = lane_u32(f2, __builtin_ctzll(left));
+                const uint32_t c = lane_word(f2, __builtin_ctzll(left));
                 const uint64_t here = __ballot(f2 == c);
                 left &= ~here;
                 if (!__ballot(col == c)) {
@@ -300,7 +297,7 @@ __global__ __launch_bounds__(kBlock) void k_ls_wave(
             continue;
         }
         uint32_t at = 0;
-        for (uint32_t i = 0; i < ncol; ++i) at += lane_u32(col, int(i)) < col ? 1u : 0u;
+        for (uint32_t i = 0; i < ncol; ++i) at += lane_word(col, int(i)) < col ? 1u : 0u;
         if (uint32_t(lane) < ncol) {
             const uint32_t j = rowptr[f] + at;
             colind[j] = col;

@@ -96,8 +96,11 @@ __device__ __forceinline__ void column_partials_v(const T (&v)[V], uint32_t k, u
 
 // Columns per lane of the row-group SpMM kernels for k right-hand sides
 // (G = k rounded up to a power of two lanes per row with one): two, gathered
-// as one 16-byte copy per entry, for FP64 when k is even and at least 6 (4-8 %
-// faster FP64 solves; FP32 pairs, 8 bytes, measured no faster).
+// as one 16-byte copy per entry, for FP64 when k is even and at least 6.  FP64
+// solves (cotangent grids, t = 1), one column per lane -> two: 300^2 k = 8 2.41 ->
+// 2.42 ms, k = 32 4.42 -> 3.92; 700^2 5.51 -> 5.18, 17.8 -> 14.9; 1500^2 20.2 -> 17.9,
+// 79.6 -> 66.7.  FP32 keeps one: pairs (8 bytes) take mixed solves from 3.16 to
+// 3.56 ms (300^2, k = 8), 5.11 to 5.30 (700^2), but 18.2 to 16.7 at 1500^2.
 template <typename T>
 bool multi_two_cols(uint32_t k) {
     return std::is_same<T, double>::value && k % 2 == 0 && k >= 6;
