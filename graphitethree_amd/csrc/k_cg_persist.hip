@@ -23,9 +23,8 @@
 // 9.0 us instead of 4.3).
 //
 // The launch is not cooperative: it uses at most one workgroup of 512 threads
-// per CU, which one always holds, at most one such launch runs at a time in a
-// process (the caller's
-// lock), and every wait is bounded.  A workgroup that gives up sets
+// per CU, which one always holds, one such launch runs at a time in a process
+// (GridTurn), and every wait is bounded.  A workgroup that gives up sets
 // kPersistFail and leaves; the others then give up at the latest at the
 // barrier before the solver's vectors, partials and status are written,
 // which is complete for all or for none of them (grid_barrier.h; a wait that

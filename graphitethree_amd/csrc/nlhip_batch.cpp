@@ -161,8 +161,9 @@ void batch_loop(Batch& B, BatchWork<T>& w, bool precond, int max_iter, uint32_t 
     uint32_t pgrid = 0;
     // while another kernel with grid-wide barriers holds the device: in
     // launches, the same bits
-    std::unique_lock<std::mutex> barrier_lock(grid_barrier_mutex(), std::defer_lock);
-    const bool persistent = B.persistent && barrier_lock.try_lock();
+    GridTurn::Hold turn;
+    if (B.persistent) turn = grid_turn().take(GridTurn::Wait::Never);
+    const bool persistent = bool(turn);
     if (persistent) {
         NLHIP_CHECK(batch_persistent_grid<T>(w.args, precond, &pgrid));
         pgrid = std::min(pgrid, std::max(B.grid, 1u));

@@ -138,9 +138,9 @@ std::shared_mutex& capture_mutex() {
     return *m;
 }
 
-std::mutex& grid_barrier_mutex() {
-    static std::mutex* m = new std::mutex();  // process lifetime
-    return *m;
+GridTurn& grid_turn() {
+    static GridTurn* t = new GridTurn();  // process lifetime
+    return *t;
 }
 
 Stream::Stream() {

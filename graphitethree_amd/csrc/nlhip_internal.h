@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstdint>
 #include <cstring>
 #include <functional>
@@ -16,6 +17,7 @@
 #include <string>
 #include <vector>
 
+#include "grid_turn.h"
 #include "nl.h"
 #include "nl_hip.h"
 #include "nlhip_kernels.h"
@@ -221,9 +223,8 @@ class Event {
 
 float elapsed_ms(const Event& a, const Event& b);
 
-// Held while a kernel with grid-wide barriers may be running: two of them,
-// each partly resident, would wait for one another.
-std::mutex& grid_barrier_mutex();
+// The process's turn for kernels with grid-wide barriers (grid_turn.h).
+GridTurn& grid_turn();
 
 // ------------------------------------------------------------------ graphs
 
@@ -458,6 +459,9 @@ struct PersistUse {
     uint64_t launches = 0, given_up = 0;
     void gave_up() {
         ++given_up;
+        busy();
+    }
+    void busy() {
         backoff = backoff ? std::min(2 * backoff, kMost) : kFirst;
         skip = backoff;
     }

@@ -282,13 +282,21 @@ uint32_t auto_check_every(const System& S) {
     return uint32_t(std::clamp(2.0e-3 / iter_s, 8.0, 128.0));
 }
 
-// Iterations of one k_cg_persist launch (some 10 ms).
-constexpr uint32_t kPersistIters = 4096;
+// Iterations of one k_cg_persist launch: up to about 25 ms for systems that
+// leave other kernels some compute units, about 11 for larger ones, whose turns
+// alternate with those of other solves (0.4% of their time).
+constexpr uint32_t kPersistIters = 4096, kPersistItersWide = 1024;
+// Beside a launch that needs most of the device the three launches per
+// iteration of another solve starve, so large systems wait for their turn and
+// those of more than one XCD do when a large one is ahead (ms per solve beside
+// a thread that solves 201 k rows, in launches -> in turns: 201 k rows 1018 ->
+// 369, 24 k 60 -> 24; 1.2 k, which do not wait, 4.5).
+constexpr std::chrono::milliseconds kTurnWait{100};
 
 // Runs a started CG (arguments set, status open) with many iterations per
 // launch until its loop has stopped (the status in fin).  False where the
 // system is not of that kind (the first launch looks at its rows), another
-// such kernel holds the device, or a grid-wide wait was given up, now or a short while ago (PersistUse): the
+// such kernel has the turn, or a grid-wide wait was given up, now or a short while ago (PersistUse): the
 // state is then where the captured iterations, which form the same sums,
 // continue.
 template <typename T>
@@ -303,14 +311,22 @@ static bool run_persist(System& S, CGWorkspace<T>& ws, CGStatus<T>& fin) {
         --use.skip;
         return false;
     }
-    std::unique_lock<std::mutex> lock(grid_barrier_mutex(), std::try_to_lock);
-    if (!lock.owns_lock()) return false;
+    const bool wide = 2 * p.shape.wgs > uint32_t(std::max(0, device().cu_count));
+    const GridTurn::Wait wait = wide                  ? GridTurn::Wait::Large
+                                : p.shape.stride == 1 ? GridTurn::Wait::ForLarge
+                                                      : GridTurn::Wait::Never;
+    auto take = [&] { return grid_turn().take(wait, kTurnWait); };
+    GridTurn::Hold turn = take();
+    if (!turn) {
+        if (wide) use.busy();
+        return false;
+    }
     hipStream_t s = S.stream.get();
     ws.dh.ensure(2 * size_t(S.n));
     ws.slots.ensure(persist_slot_words<T>(ws.args.P));
     ws.bar.ensure(9 * kPersistBarPad);
     ws.bar_host.ensure(1);
-    p.n_iter = kPersistIters;
+    p.n_iter = wide ? kPersistItersWide : kPersistIters;
     p.polls = use.polls;
     p.sum_polls = use.sum_polls;
     p.dh = ws.dh.get();
@@ -332,6 +348,9 @@ static bool run_persist(System& S, CGWorkspace<T>& ws, CGStatus<T>& fin) {
             return false;
         }
         if (host[0].done) break;
+        turn = GridTurn::Hold();  // others that wait come first
+        turn = take();
+        if (!turn) return false;
     }
     use.backoff = 0;
     fin = host[0];

@@ -242,3 +242,42 @@ def test_systems_of_long_rows_keep_to_the_launches(hip, n, d, pairs, taken):
     x2, _ = S.solve(b, confirm=0)
     assert np.array_equal(x, x2) and S.persist_info() == (2 if taken else 1, 0)
     S.close()
+
+
+def test_large_solves_take_turns(hip):
+    """Two threads with a system that needs most of the device each, and one
+    with a medium one: all keep to launches of many iterations, in turns, with
+    the bits of a solve alone (in three launches per iteration beside a large
+    one's they would starve)."""
+    import threading
+
+    Sw = W.lscm_grid(317, seed=1)
+    x0, _ = capi.System.from_crs(Sw).solve(Sw.b, max_iter=6000, confirm=0)
+    S = [capi.System.from_crs(Sw) for _ in range(2)]
+    Mw = random_spd(20000, 6, 3, wrap=True)
+    M = capi.System.from_crs(Mw)
+    m0, _ = M.solve(Mw.b, confirm=0)
+    go = threading.Barrier(3)
+    got = [[], [], []]
+
+    def run(i):
+        go.wait()
+        for _ in range(3):
+            got[i].append(S[i].solve(Sw.b, max_iter=6000, confirm=0)[0])
+
+    def run_medium():
+        go.wait()
+        for _ in range(10):
+            got[2].append(M.solve(Mw.b, confirm=0)[0])
+
+    t = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+    t.append(threading.Thread(target=run_medium))
+    [x.start() for x in t]
+    [x.join() for x in t]
+    for i in range(2):
+        assert len(got[i]) == 3 and all(np.array_equal(x, x0) for x in got[i])
+        assert S[i].persist_info() == (3 * 6, 0)  # of 1024 iterations each
+        S[i].close()
+    assert len(got[2]) == 10 and all(np.array_equal(x, m0) for x in got[2])
+    assert M.persist_info() == (11, 0)
+    M.close()

@@ -1,6 +1,6 @@
 """The launches of many PCG iterations, on the host: the give-up protocol of
 their grid barrier (csrc/grid_barrier.h), every access a scheduling point of a
-model, and their choice (csrc/persist_plan.h)."""
+model, their choice (csrc/persist_plan.h) and their turns (csrc/grid_turn.h)."""
 import os
 import subprocess
 
@@ -11,7 +11,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 def build(tmp_path_factory, name):
     out = str(tmp_path_factory.mktemp("protocol") / name)
-    r = subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror",
+    r = subprocess.run(["g++", "-std=c++17", "-O1", "-pthread", "-Wall", "-Wextra", "-Werror",
                         "-I" + os.path.join(ROOT, "graphitethree_amd", "csrc"),
                         os.path.join(ROOT, "tests", "protocol", name + ".cpp"), "-o", out],
                        stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
@@ -45,3 +45,9 @@ def test_workgroups_that_wait_for_one_another_are_resident(tmp_path_factory):
                        text=True, timeout=100)
     assert r.returncode == 0, r.stdout
     assert int(r.stdout.split()[3]) > 0
+
+
+def test_turns_go_in_order_to_one_holder_at_a_time(tmp_path_factory):
+    r = subprocess.run([build(tmp_path_factory, "grid_turn")], stdout=subprocess.PIPE, text=True,
+                       timeout=100)
+    assert r.returncode == 0, r.stdout
