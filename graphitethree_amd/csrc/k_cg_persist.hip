@@ -303,9 +303,8 @@ __global__ __launch_bounds__(MAXT) void k_cg_persist(CGArgs<T> a, CGPersist<T> p
                 const uint32_t i = k + uint32_t(lane);
                 T t[N];
                 bool good = false;
-                for (uint32_t polls = 0; !good; ++polls) {
+                for (uint32_t polls = 0;; ++polls) {
                     good = true;
-                    const uint32_t limit = *static_cast<volatile uint32_t*>(&s_polls[1]);
 #pragma unroll
                     for (int q = 0; q < N; ++q) {
                         t[q] = T(0);
@@ -314,7 +313,8 @@ __global__ __launch_bounds__(MAXT) void k_cg_persist(CGArgs<T> a, CGPersist<T> p
                                                    tag, t[q]);
                     }
                     good = __all(good);
-                    if (polls >= limit) {
+                    if (good) break;
+                    if (polls >= *static_cast<volatile uint32_t*>(&s_polls[1])) {
                         s_ok = 0;
                         break;
                     }
@@ -348,6 +348,12 @@ __global__ __launch_bounds__(MAXT) void k_cg_persist(CGArgs<T> a, CGPersist<T> p
     for (int e = 0; e < E; ++e)
         if (in[e]) dh.store(kPair * ri[e], d[e], h[e]);
     if (!barrier()) return;
+    // no polls at all (a test): one sum is missing, whoever else polls first
+    if (p.sum_polls == 0 && gw == 0) {
+        if (threadIdx.x == 0)
+            __hip_atomic_fetch_or(p.bar, kPersistFail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return;
+    }
     // r.h and r.r of the current state, from the previous launch's partials
     for (uint32_t v = threadIdx.x / kWave; v < 4; v += blockDim.x / kWave) {
         T s0 = T(0), s1 = T(0);
