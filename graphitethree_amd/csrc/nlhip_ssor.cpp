@@ -25,19 +25,26 @@ constexpr uint64_t kChainLoads = 9000;
 
 // level(i) = 1 + the deepest level among the rows i reads (j < i for the
 // forward sweep, j > i for the backward one); rows counting-sorted by level
-// (increasing row index within a level).
+// (increasing row index within a level); eoff: the first of the entries that
+// each position reads.
 void level_schedule(uint32_t n, const std::vector<uint32_t>& rp, const std::vector<uint32_t>& ci,
-                    bool upper, std::vector<uint32_t>& rows, std::vector<uint32_t>& off) {
+                    bool upper, std::vector<uint32_t>& rows, std::vector<uint32_t>& off,
+                    std::vector<uint32_t>& eoff) {
+    std::vector<uint32_t> reads(n);
     std::vector<uint32_t> lev(n, 0);
     uint32_t top = 0;
     for (uint32_t k = 0; k < n; ++k) {
         const uint32_t i = upper ? n - 1 - k : k;
-        uint32_t l = 0;
+        uint32_t l = 0, m = 0;
         for (uint32_t e = rp[i]; e < rp[i + 1]; ++e) {
             const uint32_t j = ci[e];
-            if (upper ? j > i : j < i) l = std::max(l, lev[j] + 1);
+            if (upper ? j > i : j < i) {
+                l = std::max(l, lev[j] + 1);
+                ++m;
+            }
         }
         lev[i] = l;
+        reads[i] = m;
         top = std::max(top, l);
     }
     off.assign(size_t(top) + 2, 0);
@@ -46,6 +53,8 @@ void level_schedule(uint32_t n, const std::vector<uint32_t>& rp, const std::vect
     rows.resize(n);
     std::vector<uint32_t> next(off.begin(), off.end() - 1);
     for (uint32_t i = 0; i < n; ++i) rows[next[lev[i]]++] = i;
+    eoff.assign(size_t(n) + 1, 0);
+    for (uint32_t k = 0; k < n; ++k) eoff[k + 1] = eoff[k] + reads[rows[k]];
 }
 
 }  // namespace
@@ -123,15 +132,8 @@ namespace {
 std::vector<Ssor::Step> build_sweep(uint32_t n, const std::vector<uint32_t>& rp,
                                     const std::vector<uint32_t>& ci, const std::vector<double>& va,
                                     bool upper, SweepBufs& B, hipStream_t s) {
-    std::vector<uint32_t> rows, off;
-    level_schedule(n, rp, ci, upper, rows, off);
-    std::vector<uint32_t> eoff(size_t(n) + 1, 0);
-    for (uint32_t k = 0; k < n; ++k) {
-        const uint32_t i = rows[k];
-        uint32_t m = 0;
-        for (uint32_t e = rp[i]; e < rp[i + 1]; ++e) m += (upper ? ci[e] > i : ci[e] < i) ? 1u : 0u;
-        eoff[k + 1] = eoff[k] + m;
-    }
+    std::vector<uint32_t> rows, off, eoff;
+    level_schedule(n, rp, ci, upper, rows, off, eoff);
     std::vector<Ssor::Step> steps = plan(off, eoff);
     // columns for the levels launched over the grid, positions for the others
     bool by_col = false, by_pos = false;
